@@ -64,12 +64,15 @@ struct NormArgs {
 
 constexpr int kRowsPerBlock = 4;  // one wave per row
 // Rows are read once and written once: non-temporal loads and stores.
-// Measured at the Qwen3-8B shape (fused add, T 8192, hidden 4096) on
-// buffers rotated past the 256 MB last-level cache: 4.62 -> 5.38 TB/s; the
-// same rows re-run back to back from the cache lose 6.5 -> 5.6 TB/s.
 constexpr bool kNormNt = true;
+// Rows of 513 to 1024 elements (two waves) keep a wave per row when there are
+// many: 4096 rows 7.3 us against 7.5, 8192 rows 12.1 against 12.9; the
+// workgroup per row wins at 3000 rows (5.6 against 6.6) and below.
+constexpr int64_t kShortRowsByWave = 3500;
 
-// One wave per row. NV > 0: the row (<= 512 NV elements) stays in registers
+// One wave per row, for rows of at most 512 elements, many rows of at most
+// 1024, and rows longer than 8192 (what lies between takes the workgroup-per-row
+// kernel below). NV > 0: the row (<= 512 NV elements) stays in registers
 // between the sum of squares and the scaling, so HBM sees one read and one
 // write. NV == 0: rows longer than 8192 elements take a second pass that
 // re-reads the row (for the fused add, the rounded sum it wrote to residual).
@@ -141,6 +144,57 @@ __global__ void __launch_bounds__(kWave * kRowsPerBlock) rmsnorm_kernel(NormArgs
   }
 }
 
+// One workgroup per row, one 16-byte chunk per thread (blockDim.x = d / 8 in
+// whole waves, rows of at most 8192 elements). What bounds the call is the
+// latency of one pass over the row for a decode batch and HBM's mixed
+// read/write rate for a prefill batch; both want every load of the row (x,
+// residual, weight) issued at once by as many waves as the row has, not a
+// lane walking its share of the row. Then one wave sum, one exchange of the
+// wave sums through LDS, and the store.
+// Fused add, hidden 4096, us per call in a captured graph on rotated buffers,
+// a wave per row -> a workgroup per row: 64 rows 10.0 -> 2.7, 1024 13.0 -> 7.5,
+// 2048 16.1 -> 13.0, 8192 51 -> 44.5 (6.0 TB/s); non-temporal accesses against
+// cached ones here: 7.5 against 9.0 at 1024 rows, 44.5 against 49.8 at 8192.
+template <int DT, bool VEC, bool ADD>
+__global__ void __launch_bounds__(1024) rmsnorm_row_kernel(NormArgs a) {
+  __shared__ float part[16];
+  const int64_t row = blockIdx.x;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t e0 = static_cast<int64_t>(threadIdx.x) * 8;
+  uint16_t* xr = a.x + row * a.x_st;
+  uint16_t* outr = ADD ? xr : a.out + row * a.out_st;
+  float f[8], w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f[i] = w[i] = 0.f;
+  if (e0 < a.d) {
+    load8<DT, VEC, kNormNt>(xr, e0, a.d, f);
+    load8<DT, VEC>(a.w, e0, a.d, w);
+    if constexpr (ADD) {
+      uint16_t* rr = a.residual + row * a.r_st;
+      float r[8];
+      load8<DT, VEC, kNormNt>(rr, e0, a.d, r);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) f[i] += r[i];
+      store8<DT, VEC, kNormNt>(rr, e0, a.d, f);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ss += f[i] * f[i];
+  ss = wave_sum(ss);
+  if (lane == 0) part[wave] = ss;
+  __syncthreads();
+  const int nwaves = blockDim.x >> 6;
+  ss = 0.f;
+  for (int i = 0; i < nwaves; ++i) ss += part[i];
+  const float scale = 1.0f / sqrtf(ss / static_cast<float>(a.d) + a.eps);
+  if (e0 < a.d) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = (f[i] * scale) * w[i];
+    store8<DT, VEC, kNormNt>(outr, e0, a.d, f);
+  }
+}
+
 struct ActArgs {
   uint16_t* out;
   const uint16_t* in;
@@ -166,8 +220,7 @@ __device__ __forceinline__ float act_mul(float x, float y) {
 // Input and output are streamed non-temporally: each element is read or
 // written once, and at Qwen3-8B's shape (8192 tokens x 12288) the 604 MB
 // pass is larger than the last-level cache, which cached accesses only
-// thrash (measured 103.4 -> 92.1 us). The norm kernels keep cached accesses:
-// their passes fit that cache and non-temporal ones measured slower there.
+// thrash (measured 103.4 -> 92.1 us).
 template <int DT, int ACT, bool VEC>
 __global__ void __launch_bounds__(256) act_and_mul_kernel(ActArgs a) {
   const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
@@ -215,11 +268,17 @@ void launch_norm_vec(bool vec, const NormArgs& a, hipStream_t s) {
 template <int DT, bool ADD>
 void launch_norm(bool vec, const NormArgs& a, hipStream_t s) {
   const int64_t chunks = (a.d + 511) / 512;
+  const bool by_wave = chunks <= 1 || (chunks == 2 && a.rows > kShortRowsByWave);
+  if (!by_wave && chunks <= 16 && a.rows <= 0x7fffffff) {
+    const dim3 grid(static_cast<uint32_t>(a.rows)), block(static_cast<uint32_t>(chunks) * kWave);
+    if (vec)
+      hipLaunchKernelGGL((rmsnorm_row_kernel<DT, true, ADD>), grid, block, 0, s, a);
+    else
+      hipLaunchKernelGGL((rmsnorm_row_kernel<DT, false, ADD>), grid, block, 0, s, a);
+    return;
+  }
   if (chunks <= 1) launch_norm_vec<DT, 1, ADD>(vec, a, s);
   else if (chunks <= 2) launch_norm_vec<DT, 2, ADD>(vec, a, s);
-  else if (chunks <= 4) launch_norm_vec<DT, 4, ADD>(vec, a, s);
-  else if (chunks <= 8) launch_norm_vec<DT, 8, ADD>(vec, a, s);
-  else if (chunks <= 16) launch_norm_vec<DT, 16, ADD>(vec, a, s);
   else launch_norm_vec<DT, 0, ADD>(vec, a, s);
 }
 

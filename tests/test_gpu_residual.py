@@ -173,3 +173,28 @@ def test_residual_path_rejects_bad_arguments(dev):
                                w.to(torch.bfloat16), 1e-6)
     with pytest.raises(ValueError):
         capi.silu_and_mul(torch.empty((4, 31), device=dev, dtype=torch.bfloat16), xb)
+
+
+@pytest.mark.parametrize("dtype", ["bf16", "fp16"])
+@pytest.mark.parametrize("rows,d", [
+    (2, 512), (2, 513), (1, 520), (3, 1023),  # a wave per row / two waves
+    (3500, 1024), (3501, 1024),               # either side of the many-short-rows rule
+    (5, 1032), (1, 4088), (64, 4096), (2, 4097), (1, 8191), (3, 8192), (2, 8193),
+])
+def test_norm_kernels_at_their_limits(oracle, dev, rows, d, dtype):
+    """RMSNorm with and without the residual add where one kernel hands over
+    to the next: partly filled waves, odd widths, the longest held row."""
+    note(f"norm limits rows={rows} d={d} {dtype}")
+    x = rand_t((rows, d), dtype, dev, 5)
+    r = rand_t((rows, d), dtype, dev, 6, 3.0)
+    w = (torch.rand(d, device=dev) + 0.5).to(TORCH_DT[dtype])
+    out = capi.rmsnorm(x, w, 1e-6)
+    torch.cuda.synchronize()
+    assert_within_ulp(host(out), oracle.rmsnorm(host(x), host(w), 1e-6, dtype), dtype, "rmsnorm")
+    xo_ref, ro_ref = oracle.fused_add_rmsnorm(host(x), host(r), host(w), 1e-6, dtype)
+    capi.fused_add_rmsnorm(x, r, w, 1e-6)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(host(r), ro_ref)
+    if d > 8192:  # long rows normalise the rounded sum
+        xo_ref = oracle.rmsnorm(ro_ref, host(w), 1e-6, dtype)
+    assert_within_ulp(host(x), xo_ref, dtype, "fused add rmsnorm")
