@@ -1223,7 +1223,7 @@ extern "C" int sgl_paged_mixed(const sgl_decode_plan_t* plan, const void* q,
   if (st != SGL_OK) return st;
   // The prefill role: 8-wave items of 256 packed rows (unpaired, heavy first).
   const int64_t rows_max = static_cast<int64_t>(pre_max_qo_len) * p.group;
-  const int64_t tiles = (rows_max + 255) / 256;
+  const int64_t tiles = pf::launch_tiles((rows_max + 255) / 256, num_kv_heads);
   const int64_t items = tiles * num_kv_heads * pre_batch;
   const int upw = 8 / num_kv_heads;
   // Decode workgroups rounded to a multiple of the 8 XCDs, so the prefill
@@ -1231,6 +1231,7 @@ extern "C" int sgl_paged_mixed(const sgl_decode_plan_t* plan, const void* q,
   const int64_t dec_blocks = ((plan->num_units + upw - 1) / upw + 7) / 8 * 8;
   if (items + dec_blocks > 0x7fffffff) return SGL_ERR_INVALID_ARG;
   p.tiles_per_req = static_cast<int>(tiles);
+  p.batch = pre_batch;
   size_t lds = static_cast<size_t>(upw) * unit_lds_bytes<true>(num_kv_heads, plan->kv_chunk_size);
   if (lds < static_cast<size_t>(pf::prefill_lds_bytes<8, 1>()))
     lds = pf::prefill_lds_bytes<8, 1>();

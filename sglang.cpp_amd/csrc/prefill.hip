@@ -91,11 +91,11 @@ extern "C" int sgl_paged_prefill(const void* q, int64_t q_stride_token, int64_t 
   const bool split_kv = !wide && ((rows_max + 63) / 64) * num_kv_heads * batch_size <=
                                      static_cast<int64_t>(device_cus());
   const int bm = wide ? 256 : split_kv ? 64 : 128;
-  const int64_t tiles = pair ? pairs : (rows_max + bm - 1) / bm;
+  const int64_t tiles = pair ? pairs : launch_tiles((rows_max + bm - 1) / bm, num_kv_heads);
   const int64_t items = tiles * num_kv_heads * batch_size;
   if (items > 0x7fffffff) return SGL_ERR_INVALID_ARG;
   a.tiles_per_req = static_cast<int>(tiles);
-  a.num_kv_heads = num_kv_heads;
+  a.batch = batch_size;
   const dim3 grid(static_cast<uint32_t>(items));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (pair)

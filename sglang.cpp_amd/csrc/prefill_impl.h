@@ -32,8 +32,9 @@ struct PrefillArgs {
   float scale_log2;
   uint16_t* o;
   int64_t o_st, o_sh;
-  int tiles_per_req;  // query tiles per (request, kv head)
+  int tiles_per_req;  // query tiles (or pairs) per (request, kv head), see launch_tiles
   int num_kv_heads;
+  int batch;
 };
 
 // LDS reads of the tile loop are inline asm with compile-time offsets, and
@@ -301,21 +302,26 @@ __device__ __forceinline__ void pv_steps(const LaneAddr& la, const bf16x8_t (&po
 // gather traffic per row) and one workgroup per CU, where waves w and w + 4
 // share SIMD w % 4.
 //
-// Work item w = (request, kv head, query-tile position), head-major. The
-// rows of a request form query tiles (G heads of each token packed
+// The rows of a request form query tiles (G heads of each token packed
 // row-wise), and tile i sees about (prefix + i) kv tiles. Workgroups are
-// dealt to the 8 XCDs round-robin by linear id, so when the count allows,
-// XCD x takes the contiguous share [x S, (x + 1) S), S = N / 8: the tiles of
-// one kv head stay on one or two XCDs, whose L2 then holds that head's K/V.
+// dealt to the 8 XCDs round-robin by linear id.
 //
-// kPair = false: one 32 W-row tile per item. Positions alternate between the
-// heavy and the light end (T-1, 0, T-2, 1, ...), so every share carries about
-// the same work; inside a share the heavy half is dispatched first, heaviest
-// first, then the light half, heaviest first. Suits launches of several
+// kPair = false: one 32 W-row tile per item (item_of). Every request's tiles
+// of one kv head go to the same 8 / Hkv XCDs (for head counts that divide 8
+// or are a multiple of it), dealt between them tile by tile: the heads carry
+// the same work, so the XCDs do too however ragged the requests are, and an
+// XCD's L2 holds one head's K/V. Inside an XCD the requests follow each
+// other, each with its last tiles, which see the most kv tokens, first: the
+// tiles in flight then share one or two requests' K/V in L2 (every request's
+// heaviest tiles at a time: 180 us below). Suits launches of several
 // workgroups per CU, which the dispatcher balances.
+// Giving each XCD a contiguous share of the (request, head, tile) list left
+// the XCDs of the long requests working alone: 12 prompts of 31 to 1500
+// tokens, 32q/8kv, 224 -> 167 us a layer (its store, 43 us, included).
 //
-// kPair = true (W = 8, at most one workgroup per CU): item p takes the
-// 16 W-row tiles T - 1 - p (waves 0-3) and p (waves 4-7), so every item
+// kPair = true (W = 8, at most one workgroup per CU): items are numbered
+// head-major, XCD x taking the contiguous share [x S, (x + 1) S) of them; item
+// p takes the 16 W-row tiles T - 1 - p (waves 0-3) and p (waves 4-7), so every item
 // carries the same work and each SIMD holds one heavy and one light wave.
 // Both groups share each gathered K/V tile; a group whose rows can no
 // longer see the current tile skips its compute for that step.
@@ -343,6 +349,34 @@ constexpr int prefill_lds_bytes() {
   return ring > xch ? ring : xch;
 }
 
+// Query tiles per (request, kv head) an unpaired launch is laid out for: the
+// longest request's, in whole rounds of the XCDs that share a head.
+inline int64_t launch_tiles(int64_t tiles, int num_kv_heads) {
+  const int64_t m = num_kv_heads < kXcds && kXcds % num_kv_heads == 0 ? kXcds / num_kv_heads : 1;
+  return (tiles + m - 1) / m * m;
+}
+
+// Request, kv head and query tile of item `lin` of an unpaired launch
+// (batch x Hkv x tiles_per_req items).
+__device__ __forceinline__ void item_of(const PrefillArgs& a, int lin, int& r, int& h, int& tile) {
+  const int H = a.num_kv_heads, T = a.tiles_per_req;
+  if (H < kXcds && kXcds % H == 0) {
+    const int m = kXcds / H;  // XCDs per head, consecutive ones
+    const int x = lin % kXcds, j = lin / kXcds;
+    r = j / (T / m);
+    const int rank = j - r * (T / m);
+    h = x / m;
+    tile = T - 1 - (rank * m + x % m);
+  } else {
+    // Multiples of 8 heads: head h on XCD h % 8. Other counts: the same
+    // order, the heads wherever they fall.
+    const int j = lin / H;
+    r = j / T;
+    h = lin - j * H;
+    tile = T - 1 - (j - r * T);
+  }
+}
+
 template <int W, bool kPair, int KS>
 __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int lin,
                                              int n_items) {
@@ -352,18 +386,17 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   static_assert(GW * KS == W && (GW == 2 || GW == 4 || GW == 8),
                 "gather lane bases need row % 16 to take at most two values per lane");
   constexpr int kGM = kPair ? 16 * W : 32 * GW;  // rows per group tile
-  int w = lin;
-  if (kPair) {
+  int r, h, pos;  // pos: the query tile, or the pair's number
+  if constexpr (kPair) {
+    int w = lin;
     if (n_items % kXcds == 0) w = (lin % kXcds) * (n_items / kXcds) + lin / kXcds;
-  } else if (n_items % (2 * kXcds) == 0) {
-    const int share = n_items / kXcds;
-    const int j = lin / kXcds;
-    w = (lin % kXcds) * share + (j < share / 2 ? 2 * j : 2 * (share - 1 - j) + 1);
+    const int per_req = a.tiles_per_req * a.num_kv_heads;
+    r = w / per_req;
+    h = (w - r * per_req) / a.tiles_per_req;
+    pos = w - r * per_req - h * a.tiles_per_req;
+  } else {
+    item_of(a, lin, r, h, pos);
   }
-  const int per_req = a.tiles_per_req * a.num_kv_heads;
-  const int r = w / per_req;
-  const int h = (w - r * per_req) / a.tiles_per_req;
-  const int pos = w - r * per_req - h * a.tiles_per_req;
   const int qo_len = a.qo_indptr[r + 1] - a.qo_indptr[r];
   const int qo_beg = a.q_start ? a.q_start[r] : a.qo_indptr[r];
   const int kv_beg = a.kv_indptr[r];
@@ -372,8 +405,8 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   const int rows = qo_len * G;
   if (kv_len <= 0) {
     // No visible token: zero output rows, as the decode path writes for an
-    // empty request. The item at position 0 of each (request, kv head)
-    // writes the G heads of that kv head for every query token.
+    // empty request. Tile (or pair) 0 of each (request, kv head) writes the G
+    // heads of that kv head for every query token.
     if (pos == 0)
       for (int e = threadIdx.x; e < rows * (kD / 8); e += blockDim.x) {
         const int prow = e / (kD / 8);
@@ -405,7 +438,7 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
     row0 = (grp == 0 ? tile0 : pos) * kGM;
     gwave = wave % (W / 2);
   } else {
-    tile0 = (pos & 1) ? (pos >> 1) : a.tiles_per_req - 1 - (pos >> 1);
+    tile0 = pos;
     if (tile0 * kGM >= rows) return;
     grp_rows = true;
     row0 = tile0 * kGM;

@@ -618,6 +618,21 @@ def test_prefill_ragged(oracle, dev, hq, hkv):
     check_prefill(oracle, dev, b, hq, hkv, 22, f"prefill ragged {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("hq,hkv", [(8, 1), (16, 2), (16, 4), (24, 8), (16, 16), (12, 6), (6, 3)])
+def test_prefill_every_tile_once(oracle, dev, hq, hkv):
+    """Each (request, kv head, query tile) is some workgroup's, whatever the
+    head count (dividing 8, a multiple of 8, neither) and however the tiles
+    fall into the XCDs' rounds: one tile, its edges, odd counts (the output
+    starts as NaN)."""
+    note(f"prefill tiles hq={hq} hkv={hkv}")
+    g = hq // hkv
+    edge = 128 // g  # tokens of a 128-row tile
+    lens = [1, edge - 1 or 1, edge, edge + 1, 3 * edge + 5, 700, 2, 9 * edge]
+    b = wl.make_paged_batch(np.random.default_rng(hkv), [0, 3, 0, 64, 7, 0, 0, 1],
+                            [n + c for n, c in zip(lens, [0, 3, 0, 64, 7, 0, 0, 1])], page_size=16)
+    check_prefill(oracle, dev, b, hq, hkv, 23, f"prefill tiles {hq}/{hkv}")
+
+
 @pytest.mark.parametrize("hq,hkv,qo_last", [(16, 8, 100), (32, 4, 32)])
 def test_prefill_split_kv_short_shares(oracle, dev, hq, hkv, qo_last):
     """Launches that leave CUs idle (at most one 64-row item per CU) split
