@@ -40,7 +40,7 @@ const char* sgl_status_string(int status);
 
 /* Library version, to check that the loaded .so matches this header. */
 int sgl_abi_version(void);
-#define SGL_ABI_VERSION 15
+#define SGL_ABI_VERSION 16
 
 /* ------------------------------------------------------------------ */
 /* KV-cache store                                                      */
@@ -352,6 +352,47 @@ int sgl_paged_prefill(const void* q, int64_t q_stride_token,
                       int num_kv_heads, int head_dim, float sm_scale, void* o,
                       int64_t o_stride_token, int64_t o_stride_head,
                       void* stream);
+
+/*
+ * Prefill with the lengths known on the host, for batches with too few query
+ * tiles to fill the device (a few new tokens behind long cached prefixes):
+ * the kv ranges are cut into shares that run on separate workgroups and are
+ * folded by a second launch.
+ *   sgl_prefill_plan: from the host copies of qo_indptr and kv_indptr. Writes
+ *     the launch's list into items (capacity int32 entries, at most
+ *     SGL_PREFILL_PLAN_INTS are used) and its
+ *     sizes into plan; num_items 0 when sgl_paged_prefill serves the batch at
+ *     least as well.
+ *   sgl_paged_prefill_planned: as sgl_paged_prefill for the lengths the plan
+ *     was made from; items is the device copy of the list (num_items +
+ *     num_merges entries of four int32), workspace (plan->workspace_bytes,
+ *     16-byte aligned) holds the shares' fp32 states. Calls that share a
+ *     workspace must be stream-ordered.
+ * Replaces: the PrefillPlan / split-KV scheduling of FlashInfer behind
+ *           BatchPrefillWithPagedKVCacheDispatched
+ *           (src/attention/flashinfer_backend.cu:596-679).
+ */
+typedef struct {
+  int32_t num_items;   /* workgroups per kv head */
+  int32_t num_merges;  /* query tiles folded from several shares */
+  int32_t num_qo_heads;
+  int32_t num_kv_heads;
+  int32_t head_dim;
+  int32_t reserved;
+  int64_t workspace_bytes;
+} sgl_prefill_plan_t;
+#define SGL_PREFILL_PLAN_INTS 4096
+int sgl_prefill_plan(const int32_t* qo_indptr_host, const int32_t* kv_indptr_host,
+                     int batch_size, int num_qo_heads, int num_kv_heads, int head_dim,
+                     sgl_prefill_plan_t* plan, int32_t* items, int64_t capacity);
+int sgl_paged_prefill_planned(const sgl_prefill_plan_t* plan, const int32_t* items, const void* q,
+                              int64_t q_stride_token, int64_t q_stride_head, const void* k_cache,
+                              const void* v_cache, int64_t kv_stride_slot, int64_t kv_stride_head,
+                              const int32_t* indices, const int32_t* qo_indptr,
+                              const int32_t* kv_indptr, const int32_t* q_start, int num_qo_heads,
+                              int num_kv_heads, int head_dim, float sm_scale, void* o,
+                              int64_t o_stride_token, int64_t o_stride_head, void* workspace,
+                              int64_t workspace_bytes, void* stream);
 
 /*
  * A mixed batch (decode rows beside prefill rows, the chunked-prefill step

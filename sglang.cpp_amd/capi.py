@@ -15,6 +15,7 @@ import os
 from pathlib import Path
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
 
 PKG_DIR = Path(__file__).resolve().parent
@@ -26,7 +27,7 @@ SGL_INDEX_I64 = 1
 SGL_DTYPE_BF16 = 0
 SGL_DTYPE_F16 = 1
 SGL_DTYPE_F32 = 2
-ABI_VERSION = 15
+ABI_VERSION = 16
 FUSED_NO_K_WRITEBACK = 1  # SGL_FUSED_NO_K_WRITEBACK
 
 
@@ -49,6 +50,22 @@ class DecodePlan(ctypes.Structure):
         ("max_total_tokens", ctypes.c_int64),
         ("workspace_bytes", ctypes.c_int64),
     ]
+
+
+class PrefillPlan(ctypes.Structure):
+    """sgl_prefill_plan_t."""
+    _fields_ = [
+        ("num_items", ctypes.c_int32),
+        ("num_merges", ctypes.c_int32),
+        ("num_qo_heads", ctypes.c_int32),
+        ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
+        ("workspace_bytes", ctypes.c_int64),
+    ]
+
+
+PREFILL_PLAN_INTS = 4096
 
 
 class I32Copy(ctypes.Structure):
@@ -107,6 +124,11 @@ _SIGNATURES = {
                                              _i32, _i32, _vp], _i32),
     "sgl_paged_prefill": ([_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i32,
                            _i32, _i32, _i32, _i32, _f32, _vp, _i64, _i64, _vp], _i32),
+    "sgl_prefill_plan": ([_vp, _vp, _i32, _i32, _i32, _i32, ctypes.POINTER(PrefillPlan), _vp,
+                          _i64], _i32),
+    "sgl_paged_prefill_planned": ([ctypes.POINTER(PrefillPlan), _vp, _vp, _i64, _i64, _vp, _vp,
+                                   _i64, _i64, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _f32, _vp,
+                                   _i64, _i64, _vp, _i64, _vp], _i32),
     "sgl_mixed_decode_cus": ([_i64, _i32, _i32, ctypes.c_double], _i32),
     "sgl_decode_plan_cus": ([_vp, _i32, _i32, _i32, _i32, _i32, ctypes.POINTER(DecodePlan)], _i32),
     "sgl_paged_mixed": ([ctypes.POINTER(DecodePlan), _vp, _i64, _i64, _vp, _vp, _i64, _i64,
@@ -584,6 +606,42 @@ def paged_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                                    max_qo_len,
                                    hq, hkv, D, scale, _p(o), o.stride(0), o.stride(1),
                                    _stream(dev)), "sgl_paged_prefill")
+
+
+def prefill_plan(qo_indptr: np.ndarray, kv_indptr: np.ndarray, num_qo_heads: int,
+                 num_kv_heads: int, head_dim: int):
+    """(plan, list) of sgl_prefill_plan for host indptrs; plan.num_items is 0 when
+    paged_prefill serves the batch at least as well."""
+    qo = np.ascontiguousarray(qo_indptr, dtype=np.int32)
+    kv = np.ascontiguousarray(kv_indptr, dtype=np.int32)
+    plan, items = PrefillPlan(), np.zeros(PREFILL_PLAN_INTS, dtype=np.int32)
+    _check(lib().sgl_prefill_plan(qo.ctypes.data, kv.ctypes.data, len(qo) - 1, num_qo_heads,
+                                  num_kv_heads, head_dim, ctypes.byref(plan), items.ctypes.data,
+                                  items.size), "sgl_prefill_plan")
+    return plan, items[:4 * (plan.num_items + plan.num_merges)].reshape(-1, 4)
+
+
+def paged_prefill_planned(plan: PrefillPlan, items: torch.Tensor, q: torch.Tensor,
+                          k_cache: torch.Tensor, v_cache: torch.Tensor, indices: torch.Tensor,
+                          qo_indptr: torch.Tensor, kv_indptr: torch.Tensor, o: torch.Tensor,
+                          workspace: torch.Tensor, sm_scale: Optional[float] = None,
+                          q_start: Optional[torch.Tensor] = None) -> None:
+    dev = _need_gpu(items, q, k_cache, v_cache, indices, qo_indptr, kv_indptr, o, workspace, q_start)
+    if q.dtype != torch.bfloat16 or k_cache.dtype != torch.bfloat16 or o.dtype != torch.bfloat16:
+        raise ValueError("prefill supports bf16 q / KV / o only")
+    if items.dtype != torch.int32 or items.numel() != 4 * (plan.num_items + plan.num_merges):
+        raise ValueError("items must be the int32 list of prefill_plan")
+    hq, D = q.shape[1], q.shape[2]
+    hkv = k_cache.shape[1]
+    ss, sh = _kv_strides(k_cache)
+    if v_cache.stride() != k_cache.stride():
+        raise ValueError("K and V caches must share strides")
+    scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
+    _check(lib().sgl_paged_prefill_planned(
+        ctypes.byref(plan), _p(items), _p(q), q.stride(0), q.stride(1), _p(k_cache), _p(v_cache),
+        ss, sh, _p(indices), _p(qo_indptr), _p(kv_indptr), _p(q_start), hq, hkv, D, scale, _p(o),
+        o.stride(0), o.stride(1), _p(workspace), workspace.numel() * workspace.element_size(),
+        _stream(dev)), "sgl_paged_prefill_planned")
 
 
 # ---------------------------------------------------------------- sampling

@@ -98,7 +98,7 @@ torch::Tensor HipAttnMetadata::get_last_indices(int bs) const {
 void HipAttnMetadata::record_stream(const c10::hip::HIPStream& stream) const {
   for (const torch::Tensor* t : {&indptr, &last_rows, &dec_kv_indptr, &dec_indices, &dec_q_rows,
                                  &dec_table_idx, &pre_qo_indptr, &pre_kv_indptr, &pre_indices,
-                                 &pre_q_start, &pre_table_idx}) {
+                                 &pre_q_start, &pre_table_idx, &pre_items}) {
     if (t->defined() && t->is_cuda() && t->numel() > 0)
       c10::hip::HIPCachingAllocator::recordStream(t->storage().data_ptr(), stream);
   }
@@ -312,6 +312,16 @@ void HipAttnBackend::prepare_metadata(Batch& batch) {
   const int64_t o_dip = up.add(dec_ip), o_drows = up.add(dec_rows);
   const int64_t o_pqo = up.add(pre_qo), o_pip = up.add(pre_ip), o_pstart = up.add(pre_start);
   const int64_t o_table = up.add(table);
+  int64_t o_items = -1;
+  if (np > 0 && !meta->fused) {
+    std::vector<int32_t> items(SGL_PREFILL_PLAN_INTS);
+    check_sgl(sgl_prefill_plan(pre_qo.data(), pre_ip.data(), np, num_qo_heads_, num_kv_heads_,
+                               head_dim_, &meta->pre_plan, items.data(),
+                               static_cast<int64_t>(items.size())),
+              "sgl_prefill_plan");
+    items.resize(4 * static_cast<size_t>(meta->pre_plan.num_items + meta->pre_plan.num_merges));
+    if (!items.empty()) o_items = up.add(items);
+  }
   int64_t o_gather_ip = o_dip;  // decode rows only
   if (np > 0 && nd == 0) o_gather_ip = o_pip;
   if (np > 0 && nd > 0) {
@@ -358,6 +368,9 @@ void HipAttnBackend::prepare_metadata(Batch& batch) {
     meta->pre_kv_indptr = field(o_pip, np + 1);
     meta->pre_q_start = field(o_pstart, np);
     meta->pre_table_idx = field(o_table + nd, np);
+    if (o_items >= 0)
+      meta->pre_items =
+          field(o_items, 4 * static_cast<int64_t>(meta->pre_plan.num_items + meta->pre_plan.num_merges));
     meta->pre_indices = field(o_ind + pre_base, std::max<int64_t>(pre_total, 1));
   }
   meta->indptr = batch.is_prefill() ? field(o_qo, bs + 1) : meta->dec_kv_indptr;
@@ -451,7 +464,19 @@ torch::Tensor HipAttnBackend::attend(const torch::Tensor& q_in, int layer_id, Ba
                                o.stride(0), o.stride(1), ws.data_ptr(), ws.numel(), stream),
               "sgl_paged_decode");
   }
-  if (meta->num_prefill > 0) {
+  torch::Tensor pre_ws;  // freed on return, after the join below
+  if (meta->num_prefill > 0 && meta->pre_plan.num_items > 0) {
+    pre_ws = torch::empty({meta->pre_plan.workspace_bytes},
+                          torch::TensorOptions().dtype(torch::kUInt8).device(q.device()));
+    check_sgl(sgl_paged_prefill_planned(
+                  &meta->pre_plan, meta->pre_items.data_ptr<int32_t>(), q.data_ptr(), q.stride(0),
+                  q.stride(1), kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1),
+                  meta->pre_indices.data_ptr<int32_t>(), meta->pre_qo_indptr.data_ptr<int32_t>(),
+                  meta->pre_kv_indptr.data_ptr<int32_t>(), meta->pre_q_start.data_ptr<int32_t>(),
+                  num_qo_heads_, num_kv_heads_, head_dim_, sm_scale, o.data_ptr(), o.stride(0),
+                  o.stride(1), pre_ws.data_ptr(), pre_ws.numel(), pre_stream),
+              "sgl_paged_prefill_planned");
+  } else if (meta->num_prefill > 0) {
     check_sgl(sgl_paged_prefill(q.data_ptr(), q.stride(0), q.stride(1), kc.data_ptr(),
                                 vc.data_ptr(), kc.stride(0), kc.stride(1),
                                 meta->pre_indices.data_ptr<int32_t>(),

@@ -72,6 +72,10 @@ struct HipAttnMetadata : public BaseAttnMetadata {
   int num_prefill = 0;
   int max_qo_len = 0;
   torch::Tensor pre_qo_indptr, pre_kv_indptr, pre_indices, pre_q_start, pre_table_idx;
+  // Shares of the prefill rows' kv ranges when their query tiles alone would
+  // leave CUs idle (num_items 0: the unplanned launch).
+  sgl_prefill_plan_t pre_plan{};
+  torch::Tensor pre_items;
 
   bool use_capture_buffers = false;
   int64_t capture_tokens = 0;  // query rows of the captured step (replays may use fewer)

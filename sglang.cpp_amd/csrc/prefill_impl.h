@@ -35,7 +35,18 @@ struct PrefillArgs {
   int tiles_per_req;  // query tiles (or pairs) per (request, kv head), see launch_tiles
   int num_kv_heads;
   int batch;
+  // Planned launches (prefill_item kList): item lin / Hkv = {request, first
+  // packed row << 4 | waves of rows, first kv tile, end kv tile | kPartial}, kv
+  // head lin % Hkv; partial items leave their state in part[lin].
+  const int32_t* items;
+  float* part;
 };
+
+constexpr int kPartial = 1 << 30;  // the item is one kv share of its query tile
+constexpr int kListRows = 256;  // rows of a planned query tile at most (8 waves)
+// A partial item's state: 64 accumulator values, the reference point and the
+// sum of each of 512 threads, value-major (whole-wave stores and loads).
+constexpr int kPartFloats = 66 * 2 * kListRows;
 
 // LDS reads of the tile loop are inline asm with compile-time offsets, and
 // their waits are explicit: the compiler's wait insertion cannot tell the
@@ -377,7 +388,15 @@ __device__ __forceinline__ void item_of(const PrefillArgs& a, int lin, int& r, i
   }
 }
 
-template <int W, bool kPair, int KS>
+// kList = true (W = 8, KS = 1): the items and their kv shares come from a
+// host plan; a tile's shares are folded by prefill_merge_kernel. A tile has
+// the rows of up to 8 waves (a request's waves spread evenly over its tiles,
+// so a step costs what its waves cost); the waves past them only gather.
+// Streaming three tiles ahead through a four-tile ring measured the same
+// (63 against 63 us for the four requests of 18 to 76 new tokens): with the
+// device full these items are bound by HBM at up to four waves of rows and
+// by the matrix cores' and LDS's step at eight.
+template <int W, bool kPair, int KS, bool kList = false>
 __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int lin,
                                              int n_items) {
   static_assert(!kPair || (W == 8 && KS == 1),
@@ -387,7 +406,20 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
                 "gather lane bases need row % 16 to take at most two values per lane");
   constexpr int kGM = kPair ? 16 * W : 32 * GW;  // rows per group tile
   int r, h, pos;  // pos: the query tile, or the pair's number
-  if constexpr (kPair) {
+  int kv_t0 = 0, kv_t1 = 0, list_rows = 0;
+  bool partial = false;
+  if constexpr (kList) {
+    static_assert(32 * W == kListRows && !kPair && KS == 1, "planned items are 256-row tiles");
+    const int e = lin / a.num_kv_heads;
+    h = lin - e * a.num_kv_heads;
+    r = a.items[4 * e];
+    pos = a.items[4 * e + 1] >> 4;
+    list_rows = 32 * (a.items[4 * e + 1] & 15);
+    kv_t0 = a.items[4 * e + 2];
+    kv_t1 = a.items[4 * e + 3];
+    partial = (kv_t1 & kPartial) != 0;
+    kv_t1 &= kPartial - 1;
+  } else if constexpr (kPair) {
     int w = lin;
     if (n_items % kXcds == 0) w = (lin % kXcds) * (n_items / kXcds) + lin / kXcds;
     const int per_req = a.tiles_per_req * a.num_kv_heads;
@@ -429,7 +461,13 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   // group, its rows and its position in the group.
   int tile0, row0, gwave;
   bool grp_rows;
-  if (kPair) {
+  if constexpr (kList) {
+    tile0 = 0;
+    if (pos >= rows) return;
+    grp_rows = true;
+    row0 = pos;
+    gwave = wave;
+  } else if (kPair) {
     const int T = (rows + kGM - 1) / kGM;
     tile0 = T - 1 - pos;
     if (tile0 < pos) return;  // past this request's pairs
@@ -448,7 +486,8 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
 
   // This lane's query row.
   const int prow = row0 + gwave * 32 + c;
-  const bool row_ok = grp_rows && prow < rows;
+  const int row_end = kList ? min(rows, row0 + list_rows) : rows;
+  const bool row_ok = grp_rows && prow < row_end;
   const int qtok = row_ok ? prow / G : 0;
   const int qhead = h * G + (row_ok ? prow - (prow / G) * G : 0);
   const int allow = row_ok ? qtok + off : kv_len - 1;  // last visible kv token
@@ -456,11 +495,13 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   // kv tiles a group needs: up to its last row's visible token. The
   // workgroup gathers group 0's range, which contains group 1's.
   auto tiles_for = [&](int r0) {
-    const int last_row = min(rows, r0 + kGM) - 1;
+    const int last_row = min(row_end, r0 + kGM) - 1;
     return (min(kv_len, last_row / G + off + 1) + kBN - 1) / kBN;
   };
-  const int ntiles = tiles_for(tile0 * kGM);
-  const int my_tiles = !kPair ? ntiles : !grp_rows ? 0 : row0 == tile0 * kGM ? ntiles : tiles_for(row0);
+  const int ntiles = tiles_for(kList ? row0 : tile0 * kGM);
+  // A wave past the request's last row only gathers.
+  const int my_tiles = !kPair ? (row0 + gwave * 32 < row_end ? ntiles : 0)
+                       : !grp_rows ? 0 : row0 == tile0 * kGM ? ntiles : tiles_for(row0);
   // First token index at which some row of the group may be masked.
   const int first_masked = row0 / G + off + 1;
 
@@ -471,9 +512,9 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   // This group's kv tiles [tb, te) and the steps every group runs (equal,
   // so the workgroup-wide barriers match).
   const int share = (ntiles + KS - 1) / KS;
-  const int tb = min(ntiles, split * share);
-  const int te = min(ntiles, tb + share);
-  const int nsteps = share;
+  const int tb = kList ? min(ntiles, kv_t0) : min(ntiles, split * share);
+  const int te = kList ? min(ntiles, kv_t1) : min(ntiles, tb + share);
+  const int nsteps = kList ? te - tb : share;
 
   const uint16_t* kbase = a.kc + static_cast<int64_t>(h) * a.kv_sh;
   const uint16_t* vbase = a.vc + static_cast<int64_t>(h) * a.kv_sh;
@@ -679,7 +720,7 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   #pragma unroll
       for (int u = 0; u < 16 / GW; ++u) sl_v[u] = sl_k[u];
       load_slots<GW>(idx, (t + 3) * kBN, kv_len, tid, sl_k);
-      if (t < te && (!kPair || t < my_tiles)) {
+      if (t < te && t < my_tiles) {
         // S(t + 1)'s first K operand reads go out before the mask / max of
         // S(t), which hides their LDS latency (K(t + 1) landed and became
         // visible at the previous step's barrier). The full wait after the
@@ -748,6 +789,19 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
   }
 
   float l = sum_xor32(rs.l);
+  if constexpr (kList) {
+    if (partial) {
+      if (row0 + gwave * 32 >= row_end) return;  // no row of this wave
+      float* pp = a.part + static_cast<int64_t>(lin) * kPartFloats + threadIdx.x;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) pp[(16 * db + v) * 64 * W] = rs.acc[db][v];
+      pp[64 * 64 * W] = rs.m;
+      pp[65 * 64 * W] = l;
+      return;
+    }
+  }
   if (!row_ok) return;
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   uint16_t* op =

@@ -2,6 +2,7 @@
 and its host-side logic (argument checks, split-KV plan) behaves — all
 without a GPU: none of these calls reaches the HIP runtime."""
 import ctypes
+import itertools
 import re
 import subprocess
 
@@ -229,3 +230,57 @@ def test_paged_decode_rejects_inconsistent_plan():
     assert lib.sgl_paged_decode(*args(plan, plan.workspace_bytes - 1)) == -3
     # output head stride not a multiple of 8 elements (16-byte row stores)
     assert lib.sgl_paged_decode(*args(plan, plan.workspace_bytes, 132)) == -4
+
+
+@pytest.mark.parametrize("hq,hkv,lens", [
+    (32, 8, [(17, 2017), (90, 12_000), (33, 5000), (64, 64)]),
+    (32, 4, [(300, 9000)]),
+    (16, 8, [(2, 40_000)]),
+    (64, 4, [(1, 5), (31, 3000), (0, 0), (65, 2111)]),
+    (16, 16, [(128, 4096 + 128)]),
+])
+def test_prefill_plan_covers_every_kv_tile_once(hq, hkv, lens):
+    qo = [0, *itertools.accumulate(q for q, _ in lens)]
+    kv = [0, *itertools.accumulate(k for _, k in lens)]
+    plan, rows = capi.prefill_plan(qo, kv, hq, hkv, 128)
+    assert plan.num_items > 0 and len(rows) == plan.num_items + plan.num_merges
+    assert plan.num_items * hkv <= 256
+    items, merges = rows[:plan.num_items].tolist(), rows[plan.num_items:].tolist()
+    seen = {}
+    for at, (r, tile, t0, t1) in enumerate(items):
+        seen.setdefault((r, tile), []).append((t0, t1 & ~(1 << 30), bool(t1 >> 30), at))
+    g = hq // hkv
+    rows_of = {}
+    for r, tile in seen:
+        rows_of.setdefault(r, []).append((tile >> 4, tile & 15))
+    for r, (q, k) in enumerate(lens):  # every packed row in one tile of at most 8 waves
+        tiles = sorted(rows_of.get(r, []))
+        assert [t[0] for t in tiles] == [32 * sum(w for _, w in tiles[:i]) for i in range(len(tiles))]
+        assert 32 * sum(w for _, w in tiles) == -(-q * g // 32) * 32
+        assert all(1 <= w <= 8 for _, w in tiles)
+    want = {(r, tile): -(-min(k, (min(q * g, (tile >> 4) + 32 * (tile & 15)) - 1) // g + k - q + 1)
+                         // 64) for r, tile in seen for q, k in [lens[r]]}
+    folded = {(r, tile): (first, n) for r, tile, first, n in merges}
+    for key, parts in seen.items():
+        assert [p[0] for p in parts] == [0] + [p[1] for p in parts[:-1]]
+        assert parts[-1][1] == want[key]
+        assert all(p[2] == (len(parts) > 1) for p in parts)
+        assert [p[3] for p in parts] == list(range(parts[0][3], parts[0][3] + len(parts)))
+        assert folded.get(key) == ((parts[0][3], len(parts)) if len(parts) > 1 else None)
+
+
+def test_prefill_plan_leaves_full_batches_alone():
+    for hq, hkv, lens in [(32, 8, [(1500, 1500)] * 12), (32, 4, [(2048, 6144)]),
+                          (16, 8, [(128, 384)] * 8), (32, 8, [(40, 30)]), (32, 8, [])]:
+        qo = [0, *itertools.accumulate(q for q, _ in lens)]
+        kv = [0, *itertools.accumulate(k for _, k in lens)]
+        plan, rows = capi.prefill_plan(qo, kv, hq, hkv, 128)
+        assert plan.num_items == plan.num_merges == len(rows) == 0
+    # a list that does not fit, lengths that run backwards
+    lib, plan, buf = capi.lib(), capi.PrefillPlan(), (ctypes.c_int32 * 8)()
+    arr = lambda *x: (ctypes.c_int32 * len(x))(*x)
+    call = lambda qo, kv, cap: lib.sgl_prefill_plan(qo, kv, 1, 32, 8, 128, ctypes.byref(plan),
+                                                    buf, cap)
+    assert call(arr(0, 20), arr(0, 9000), 8) == -3 and plan.num_items == 0
+    assert call(arr(0, -1), arr(0, 9000), 8) == -1
+    assert call(arr(0, 20), arr(0, -5), 8) == -1

@@ -633,6 +633,38 @@ def test_prefill_every_tile_once(oracle, dev, hq, hkv):
     check_prefill(oracle, dev, b, hq, hkv, 23, f"prefill tiles {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("hq,hkv,cached,new", [
+    (32, 8, [2000, 9001, 500, 0], [17, 90, 33, 40]),  # shares beside whole tiles
+    (16, 8, [4095], [2]),                             # one wave of rows
+    (32, 4, [3000, 2999], [65, 16]),                  # G 8, a tile's edge
+    (16, 16, [2048], [129]),                          # G 1, 1 row in the last tile
+    (64, 4, [1500], [40]),                            # G 16
+    (12, 6, [3333, 1], [31, 1]),                      # heads that do not divide the XCDs
+])
+def test_prefill_planned(oracle, dev, hq, hkv, cached, new):
+    """Query tiles cut into kv shares and folded, against the oracle."""
+    note(f"planned prefill hq={hq} hkv={hkv} {cached} {new}")
+    b = wl.make_paged_batch(np.random.default_rng(5), cached,
+                            [c + n for c, n in zip(cached, new)], page_size=16)
+    plan, items = capi.prefill_plan(b.qo_indptr, b.kv_indptr, hq, hkv, 128)
+    assert plan.num_merges > 0
+    kc, vc = _pool(dev, b.num_slots, hkv, 128, 6)
+    rows = int(b.qo_indptr[-1])
+    q = randn_bf16((rows, hq, 128), dev, gen(dev, 7))
+    o = torch.full((rows, hq, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+    ws = torch.full((plan.workspace_bytes // 4,), float("nan"), device=dev)
+    idx, qop, kvp = (torch.from_numpy(x).to(dev) for x in (b.indices, b.qo_indptr, b.kv_indptr))
+    capi.paged_prefill_planned(plan, torch.from_numpy(items.copy()).to(dev), q, kc, vc, idx, qop,
+                               kvp, o, ws)
+    torch.cuda.synchronize()
+    ref = oracle.prefill(u16(q), u16(kc), u16(vc), b.indices, b.qo_indptr, b.kv_indptr,
+                         1 / math.sqrt(128))
+    assert_attn_close(o.float().cpu().numpy(), ref, what="planned prefill")
+    with pytest.raises(capi.SglError):
+        capi.paged_prefill_planned(plan, torch.from_numpy(items.copy()).to(dev), q, kc, vc, idx,
+                                   qop, kvp, o, ws[:-1])
+
+
 @pytest.mark.parametrize("hq,hkv,qo_last", [(16, 8, 100), (32, 4, 32)])
 def test_prefill_split_kv_short_shares(oracle, dev, hq, hkv, qo_last):
     """Launches that leave CUs idle (at most one 64-row item per CU) split
