@@ -230,6 +230,10 @@ typedef struct {
   int64_t max_total_tokens; /* capacity: num_units * kv_chunk_size tokens per call */
   int64_t workspace_bytes;  /* 256-byte header (status word) + fp32 partials, two per unit,
                                + one int32 per unit */
+  int32_t max_request_tokens; /* longest planned request; a caller that plans a worst case it
+                                 expects to stay well below (graph capture) may set it to 0:
+                                 batches of few tokens then always take the one-launch kernel */
+  int32_t reserved;
 } sgl_decode_plan_t;
 
 /*
@@ -279,7 +283,7 @@ int sgl_decode_plan_check(const sgl_decode_plan_t* plan, const int32_t* kv_indpt
  * head, request), or per (kv head, unit) when the batch has more requests
  * than the plan has units), or one for small batches
  * (plans at the 64-token minimum unit with batch_size x Hkv workgroups at
- * most the CU count). Calls that share one workspace must be stream-ordered.
+ * most the CU count and no request longer than 800 tokens). Calls that share one workspace must be stream-ordered.
  * Replaces: BatchDecodeWithPagedKVCacheDispatched call in
  *           FlashInferBackend::forward (src/attention/flashinfer_backend.cu:553-595).
  */

@@ -49,6 +49,8 @@ class DecodePlan(ctypes.Structure):
         ("head_dim", ctypes.c_int32),
         ("max_total_tokens", ctypes.c_int64),
         ("workspace_bytes", ctypes.c_int64),
+        ("max_request_tokens", ctypes.c_int32),
+        ("reserved", ctypes.c_int32),
     ]
 
 

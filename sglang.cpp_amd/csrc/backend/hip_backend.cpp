@@ -530,6 +530,7 @@ void HipAttnBackend::init_capture_graph(int max_seq_len, const std::vector<int>&
     sgl_decode_plan_t plan;
     check_sgl(sgl_decode_plan(worst.data(), bs, num_qo_heads_, num_kv_heads_, head_dim_, &plan),
               "sgl_decode_plan");
+    plan.max_request_tokens = 0;  // replayed requests are shorter than the worst case
     cap->plans[bs] = plan;
     ws_bytes = std::max<int64_t>(ws_bytes, plan.workspace_bytes);
   }
@@ -762,6 +763,7 @@ void HipAttnBackend::prepare_mixed_for_capture(Batch& batch) {
       check_sgl(sgl_decode_plan(worst.data(), n_dec, num_qo_heads_, num_kv_heads_, head_dim_,
                                 &meta->dec_plan),
                 "sgl_decode_plan");
+    meta->dec_plan.max_request_tokens = 0;  // as in init_capture_graph
     TORCH_CHECK(meta->dec_plan.workspace_bytes <= mixed_->workspace.numel(),
                 "mixed capture workspace too small");
     meta->dec_kv_indptr = mixed_->dec_kv_indptr.slice(0, 0, n_dec + 1);

@@ -611,8 +611,8 @@ __global__ void __launch_bounds__(512, 1) mixed_attention_kernel(DecodeArgs d, p
                                   static_cast<int>(gridDim.x) - dec_blocks);
 }
 
-// Small batches (every unit at the 64-token minimum and at most one
-// workgroup per CU for each (request, kv head)): one 8-wave workgroup per
+// Small batches (every unit at the 64-token minimum, at most one workgroup per
+// CU for each (request, kv head) and no long request): one 8-wave workgroup per
 // (kv head, request), the request's tokens cut into 8 contiguous pieces, one
 // per wave, and the waves' softmax states folded through LDS by wave 0 --
 // one launch instead of decode + merge, which is what such a call is bound
@@ -623,6 +623,12 @@ __global__ void __launch_bounds__(512, 1) mixed_attention_kernel(DecodeArgs d, p
 // Each wave streams one kv head's 256-byte row slices, so K is loaded as
 // whole rows and transposed through LDS (-13% kernel time at config 1).
 constexpr int kSmallWaves = 8;
+// A request's workgroup streams about 46 GB/s of K/V, the launch pair costs
+// the same for any length: per layer (store included, 32q/8kv, one request, a
+// captured step) 11.2, 14.0, 16.9, 19.8 and 54 us here at 256, 512, 768, 1024
+// and 4096 tokens against 17.1, 17.4, 17.5, 17.6 and 18.6 us; four requests 12.3,
+// 15.1, 18.1, 21.0 and 56 against 18.1, 18.4, 18.6, 19.2 and 24.7.
+constexpr int kSmallLongest = 800;
 constexpr int kSmallStage = 8192;  // slot indices staged in LDS (longer requests read them from HBM)
 
 __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel(DecodeArgs a) {
@@ -800,6 +806,87 @@ __global__ void __launch_bounds__(kMaxGroup * (kD / 4)) decode_merge_kernel(Deco
   merge_request(a, blockIdx.x, blockIdx.y, unit_tokens(a, a.kv_indptr[a.batch]));
 }
 
+// Few requests cut into many pieces (a batch of one or a few long requests):
+// one workgroup per (query head, request). Each of its kLongGroups groups of
+// 32 lanes (4 consecutive d a lane) folds a share of the pieces, four in
+// flight at a time, and lane group 0 folds the groups through LDS. What bounds
+// it is the chain of dependent load rounds: 188 pieces are 3 rounds here and
+// 47 in the kernel above.
+constexpr int kLongGroups = 16;
+constexpr int kLongPieces = 16;  // mean pieces per request from which this kernel is used
+
+__global__ void __launch_bounds__(kLongGroups * 32) decode_merge_long_kernel(DecodeArgs a) {
+  __shared__ float xch[kLongGroups][6][32];
+  const int head = blockIdx.x, r = blockIdx.y;
+  const int lane = threadIdx.x & 31, grp = threadIdx.x >> 5;
+  const int W = unit_tokens(a, a.kv_indptr[a.batch]);
+  const int rb = a.kv_indptr[r];
+  const int re = a.kv_indptr[r + 1];
+  const int qrow = a.q_indptr ? a.q_indptr[r] : r;
+  uint16_t* op = a.o + static_cast<int64_t>(qrow) * a.o_st +
+                 static_cast<int64_t>(head) * a.o_sh + 4 * lane;
+  if (static_cast<int64_t>(re) > static_cast<int64_t>(a.num_units) * W) {
+    if (grp == 0) *reinterpret_cast<u32x2_t*>(op) = u32x2_t{0x7fc07fc0u, 0x7fc07fc0u};  // NaN
+    if (threadIdx.x == 0) *a.status = SGL_ERR_CAPACITY;  // same value from every writer
+    return;
+  }
+  if (re <= rb) return;
+  const int u0 = rb / W;
+  const int u1 = (re - 1) / W;
+  if (u0 == u1) return;  // whole request, written by the decode kernel
+  const int s0 = 2 * u0 + (rb > u0 * W ? 1 : 0);
+  const int np = u1 - u0 + 1;
+  const int per = (np + kLongGroups - 1) / kLongGroups;
+  const int c1 = min(np, (grp + 1) * per);
+  float m = -INFINITY, den = 0.f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  for (int c = grp * per; c < c1; c += kFoldPieces) {
+    float lse[kFoldPieces];
+    f32x4_t v[kFoldPieces];
+#pragma unroll
+    for (int k = 0; k < kFoldPieces; ++k) {
+      const int p = min(c + k, c1 - 1);
+      const int64_t pidx = static_cast<int64_t>(p == 0 ? s0 : 2 * (u0 + p)) * a.hq + head;
+      lse[k] = c + k < c1 ? a.part_lse[pidx] : -INFINITY;
+      v[k] = *reinterpret_cast<const f32x4_t*>(a.part_o + pidx * kD + 4 * lane);
+    }
+    float mc = m;
+#pragma unroll
+    for (int k = 0; k < kFoldPieces; ++k) mc = fmaxf(mc, lse[k]);
+    const float keep = m == -INFINITY ? 0.f : exp2f(m - mc);
+    den *= keep;
+    acc *= keep;
+    m = mc;
+#pragma unroll
+    for (int k = 0; k < kFoldPieces; ++k) {
+      const float wgt = lse[k] == -INFINITY ? 0.f : exp2f(lse[k] - m);
+      den += wgt;
+      acc += v[k] * wgt;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) xch[grp][i][lane] = acc[i];
+  xch[grp][4][lane] = m;
+  xch[grp][5][lane] = den;
+  __syncthreads();
+  if (grp != 0) return;
+  float all = -INFINITY;
+#pragma unroll
+  for (int g = 0; g < kLongGroups; ++g) all = fmaxf(all, xch[g][4][lane]);
+  float sum = 0.f, o4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int g = 0; g < kLongGroups; ++g) {
+    const float mg = xch[g][4][lane];
+    const float wgt = mg == -INFINITY ? 0.f : exp2f(mg - all);
+    sum += xch[g][5][lane] * wgt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o4[i] += xch[g][i][lane] * wgt;
+  }
+  const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+  *reinterpret_cast<u32x2_t*>(op) =
+      u32x2_t{pack_bf16x2(o4[0] * inv, o4[1] * inv), pack_bf16x2(o4[2] * inv, o4[3] * inv)};
+}
+
 // One workgroup per (kv head, unit), for batches of more requests than
 // units: the unit where a split request ends folds it (that request is the
 // one running into the unit from before, recorded by the decode), and the
@@ -947,10 +1034,11 @@ static int decode_plan_for(const int32_t* kv_indptr_host, int batch_size, int nu
   int64_t w_dev = round16((total + units - 1) / units);
   if (w_dev < kMinUnit) w_dev = kMinUnit;
   if (w_dev > W) w_dev = W;
-  int split = 0;
-  for (int r = 0; r < batch_size && !split; ++r) {
+  int split = 0, longest = 0;
+  for (int r = 0; r < batch_size; ++r) {
     const int rb = kv_indptr_host[r], re = kv_indptr_host[r + 1];
     if (re > rb && (re - 1) / w_dev != rb / w_dev) split = 1;
+    if (re - rb > longest) longest = re - rb;
   }
   plan->kv_chunk_size = static_cast<int32_t>(W);
   plan->min_chunk_size = kMinUnit;
@@ -962,6 +1050,8 @@ static int decode_plan_for(const int32_t* kv_indptr_host, int batch_size, int nu
   plan->head_dim = head_dim;
   plan->max_total_tokens = units * W;
   plan->workspace_bytes = workspace_layout(static_cast<int>(units), num_qo_heads).total;
+  plan->max_request_tokens = longest;
+  plan->reserved = 0;
   return SGL_OK;
 }
 
@@ -1106,6 +1196,9 @@ void launch_merge(const DecodeArgs& a, hipStream_t s) {
   if (a.batch > a.num_units + 1)
     hipLaunchKernelGGL(decode_merge_units_kernel, dim3(a.hkv, a.num_units + 1),
                        dim3(merge_threads(a.group)), 0, s, a);
+  else if (a.num_units >= kLongPieces * static_cast<int64_t>(a.batch))
+    hipLaunchKernelGGL(decode_merge_long_kernel, dim3(a.hq, a.batch), dim3(kLongGroups * 32), 0, s,
+                       a);
   else
     hipLaunchKernelGGL(decode_merge_kernel, dim3(a.hkv, a.batch), dim3(merge_threads(a.group)), 0,
                        s, a);
@@ -1123,7 +1216,7 @@ void bind_workspace(DecodeArgs& a, const sgl_decode_plan_t* plan, void* workspac
 
 // Decode launch + merge launch on one stream (or the small-batch kernel alone).
 int launch_decode(const DecodeArgs& a, const sgl_decode_plan_t* plan, hipStream_t s) {
-  if (plan->kv_chunk_size <= kMinUnit &&
+  if (plan->kv_chunk_size <= kMinUnit && plan->max_request_tokens <= kSmallLongest &&
       static_cast<int64_t>(a.batch) * a.hkv <= static_cast<int64_t>(device_cu_count())) {
     hipLaunchKernelGGL(paged_decode_small_kernel, dim3(a.hkv, a.batch), dim3(kSmallWaves * kWave),
                        0, s, a);

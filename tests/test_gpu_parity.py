@@ -474,6 +474,44 @@ def test_decode_small_batch_kernel(oracle, dev, hq, hkv, lens):
     assert_attn_close(o.float().cpu().numpy(), ref, what="small-batch decode")
 
 
+@pytest.mark.parametrize("unknown_longest", [False, True])
+@pytest.mark.parametrize("hq,hkv,lens", [
+    (32, 8, [800]), (32, 8, [801]),  # either side of the one-launch limit
+    (16, 8, [1024]), (16, 8, [1023, 9]),  # 16 units: the fold for few long requests, and not
+    (32, 8, [12001]), (64, 4, [5000, 3000]), (8, 8, [4097]), (8, 1, [9000]),
+])
+def test_decode_few_long_requests(oracle, dev, hq, hkv, lens, unknown_longest):
+    """One or a few long requests: many units and a fold of many pieces, or
+    (a plan that does not know the longest request) the one-launch kernel."""
+    note(f"decode few long requests hq={hq} hkv={hkv} lens={lens} {unknown_longest}")
+    rng = np.random.default_rng(31)
+    b = wl.make_paged_batch(rng, [x - 1 for x in lens], lens, page_size=16, decode=True)
+    plan = capi.decode_plan(b.kv_indptr, hq, hkv, 128)
+    assert plan.max_request_tokens == max(lens) and plan.kv_chunk_size == 64
+    if unknown_longest:
+        plan.max_request_tokens = 0
+    q, kc, vc, o, scale, _ = run_decode(dev, b, hq, hkv, 128, 32, plan=plan)
+    ref = oracle.decode(u16(q).copy(), u16(kc), u16(vc), b.indices, b.kv_indptr, scale)
+    assert_attn_close(o.float().cpu().numpy(), ref, what="few long requests")
+
+
+def test_decode_few_long_requests_past_the_plan(dev):
+    """A long request past the plan's capacity: NaN rows and the status."""
+    note("decode long request past its plan")
+    plan = capi.decode_plan(np.array([0, 2000], np.int32), 32, 8, 128)
+    assert plan.num_units >= 16
+    b = wl.make_paged_batch(np.random.default_rng(33), [plan.max_total_tokens],
+                            [plan.max_total_tokens + 1], page_size=16, decode=True)
+    kc, vc = _pool(dev, b.num_slots, 8, 128, 34)
+    q = randn_bf16((1, 32, 128), dev, gen(dev, 35))
+    o = torch.zeros_like(q)
+    ws = capi.decode_workspace(plan, dev)
+    capi.paged_decode(plan, q, kc, vc, torch.from_numpy(b.indices).to(dev),
+                      torch.from_numpy(b.kv_indptr).to(dev), o, ws, 1 / math.sqrt(128))
+    assert capi.decode_status(ws) == -3
+    assert torch.isnan(o.float()).all()
+
+
 def test_decode_plan_exceeded_reports_capacity(oracle, dev):
     """A plan reused for a longer batch: requests reaching past the plan's
     token capacity come back as NaN rows with the CAPACITY status, the others
