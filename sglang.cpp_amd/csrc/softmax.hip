@@ -161,12 +161,125 @@ __global__ void __launch_bounds__(sp::kStatLanes) softmax_temperature_held(Softm
     prow[e] = sp::prob(Elem<DT>::load1(row, e), sc, nb, inv_s);
 }
 
+// Small batches: a row's work spread over many CUs in two launches, with the
+// statistics in the same lanes, order and bits as above.
+//   softmax_lane_stats: one wave per 64 statistics lanes (16 workgroups a row)
+//     leaves the lanes' states where the probabilities will be: every slice of
+//     the row gets a copy of all 1024, so that each workgroup of the second
+//     launch reads its own and may then overwrite it.
+//   softmax_write_slices: one workgroup per slice of about 8192 elements (a
+//     16-byte chunk of 16-bit logits per thread) folds the lanes and writes.
+// With one workgroup per row a batch of 16 keeps 16 CUs busy, each with its
+// row's 900 KB; the two launches are bound by the latency of their two trips
+// to memory.
+constexpr int kSliceElems = 8 * sp::kStatLanes;
+constexpr int kLaneFloats = 2 * sp::kStatLanes;  // the copy of the lanes' states in a slice
+
+// Slices of a row: about two workgroups a CU in all (each slice costs a copy of
+// the lanes' states), of at least kSliceElems elements.
+inline int row_slices(int64_t batch, int64_t d) {
+  int64_t n = 512 / batch < 2 ? 2 : 512 / batch;
+  if (n > (d + kSliceElems - 1) / kSliceElems) n = (d + kSliceElems - 1) / kSliceElems;
+  return static_cast<int>(n);
+}
+// 16-byte chunks of a slice (the last slice takes what is left of the row).
+template <int P>
+__device__ __host__ inline int slice_chunks(int64_t d, int slices) {
+  return static_cast<int>((d / P + slices - 1) / slices);
+}
+
+template <int DT>
+__global__ void __launch_bounds__(kWave) softmax_lane_stats(SoftmaxArgs a, int slices) {
+  constexpr int P = Elem<DT>::kPer;
+  const int r = blockIdx.y;
+  const char* row = static_cast<const char*>(a.logits) + static_cast<int64_t>(r) * a.x_st * (16 / P);
+  float* prow = a.probs + static_cast<int64_t>(r) * a.p_st;
+  const int v = blockIdx.x * kWave + threadIdx.x;
+  const float sc = sp::exp2_scale(a.temps ? a.temps[r] : a.temp);
+  const sp::LaneStats st = sp::lane_stats<DT>(row, static_cast<int>(a.d), true, v, sc);
+  const int len = slice_chunks<P>(a.d, slices) * P;
+  for (int j = 0; j < slices; ++j)
+    reinterpret_cast<float2*>(prow + static_cast<int64_t>(j) * len)[v] = float2{st.mx, st.s};
+}
+
+template <int DT>
+__global__ void __launch_bounds__(sp::kStatLanes) softmax_write_slices(SoftmaxArgs a) {
+  __shared__ float red[sp::kStatWaves];
+  constexpr int P = Elem<DT>::kPer;
+  const int r = blockIdx.y, tid = threadIdx.x;
+  const char* row = static_cast<const char*>(a.logits) + static_cast<int64_t>(r) * a.x_st * (16 / P);
+  float* prow = a.probs + static_cast<int64_t>(r) * a.p_st;
+  const int d = static_cast<int>(a.d), nfull = d / P;
+  const int per = slice_chunks<P>(d, gridDim.x);
+  const int c0 = blockIdx.x * per, c1 = min(nfull, c0 + per);
+  // The first chunk and the lane's state are in flight together.
+  u32x4_t v = {0, 0, 0, 0};
+  if (c0 + tid < c1) v = ldg128(row + static_cast<int64_t>(c0 + tid) * 16);
+  const float2 lane = reinterpret_cast<const float2*>(prow + static_cast<int64_t>(c0) * P)[tid];
+  const float sc = sp::exp2_scale(a.temps ? a.temps[r] : a.temp);
+  sp::LaneStats st;
+  st.mx = lane.x;
+  st.s = lane.y;
+  const float m = sp::block_max<sp::kStatWaves>(st.mx, red);
+  const float inv_s = 1.0f / sp::block_sum<sp::kStatWaves>(sp::lane_sum_at(st, m, sc), red);
+  const float nb = sp::exp2_offset(m, sc);
+  for (int c = c0 + tid; c < c1; c += sp::kStatLanes) {
+    if (c != c0 + tid) v = ldg128(row + static_cast<int64_t>(c) * 16);
+    float p[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) p[j] = sp::prob(Elem<DT>::at(v, j), sc, nb, inv_s);
+#pragma unroll
+    for (int q = 0; q < P / 4; ++q)
+      *reinterpret_cast<f32x4_t*>(prow + static_cast<int64_t>(c) * P + 4 * q) =
+          f32x4_t{p[4 * q], p[4 * q + 1], p[4 * q + 2], p[4 * q + 3]};
+  }
+  if (blockIdx.x + 1 == gridDim.x)
+    for (int e = nfull * P + tid; e < d; e += sp::kStatLanes)
+      prow[e] = sp::prob(Elem<DT>::load1(row, e), sc, nb, inv_s);
+}
+
+// Where the two launches win: rows long enough to pay for the second launch,
+// batches small enough to leave CUs idle. bf16 on rotated buffers, us, one
+// launch -> two: 151,936 x 1 18.2 -> 8.5, x 16 21.1 -> 14.0, x 64 25.7 -> 23.2,
+// x 96 27.9 against 31.0; 65,536 x 32 11.4 -> 10.2, x 64 13.4 against 14.2;
+// 50,000 x 4 7.9 against 8.3. fp32 (read twice by one 512-thread workgroup
+// before): 151,936 x 16 36.5 -> 16.6, x 128 57.7 -> 51.0; 32,768 x 32 9.5 ->
+// 7.7, x 96 11.9 against 13.1. bf16 rows too long to hold: 200,000 x 64 42.4 ->
+// 28.0, x 160 55.1 against 58.3.
+inline bool split_rows(bool held, int64_t batch, int64_t d) {
+  return d >= (held ? 65536 : 32768) && batch * (held ? 2000 : 1500) <= d;
+}
+
+// The first launch writes into the probabilities' rows: the logits must lie
+// elsewhere (one workgroup per row takes fp32 rows in place).
+template <int DT>
+bool overlapping(const SoftmaxArgs& a) {
+  constexpr int64_t B = 16 / Elem<DT>::kPer;
+  const uintptr_t p = reinterpret_cast<uintptr_t>(a.probs);
+  const uintptr_t x = reinterpret_cast<uintptr_t>(a.logits);
+  return p < x + static_cast<uintptr_t>(((a.batch - 1) * a.x_st + a.d) * B) &&
+         x < p + static_cast<uintptr_t>(((a.batch - 1) * a.p_st + a.d) * 4);
+}
+
 template <int DT>
 int launch_softmax(const SoftmaxArgs& a, hipStream_t s) {
   constexpr int P = Elem<DT>::kPer;
   const int64_t per_lane = (a.d / P + sp::kStatLanes - 1) / sp::kStatLanes;  // chunks per lane
   const dim3 grid(static_cast<uint32_t>(a.batch));
   const dim3 held(sp::kStatLanes);
+  const bool reg_rows = DT != SGL_DTYPE_F32 && per_lane <= kMaxRegChunks;
+  if (a.vec && a.batch <= 0xffff && split_rows(reg_rows, a.batch, a.d) &&
+      !overlapping<DT>(a)) {
+    const int slices = row_slices(a.batch, a.d);
+    hipLaunchKernelGGL((softmax_lane_stats<DT>),
+                       dim3(sp::kStatWaves, static_cast<uint32_t>(a.batch)), dim3(kWave), 0, s, a,
+                       slices);
+    const int st = launch_status();
+    if (st != SGL_OK) return st;
+    hipLaunchKernelGGL((softmax_write_slices<DT>),
+                       dim3(slices, static_cast<uint32_t>(a.batch)), held, 0, s, a);
+    return launch_status();
+  }
   if constexpr (DT == SGL_DTYPE_F32) {
     hipLaunchKernelGGL((softmax_temperature_stream<DT>), grid, dim3(kSmThreads), 0, s, a);
     return launch_status();

@@ -510,3 +510,34 @@ def test_sampler_entry_points_replay_in_a_graph(dev):
         assert torch.equal(probs, p_eager)
         assert torch.equal(s_g, s_e) and torch.equal(ok_g, ok_e)
     del graph
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("vocab", [65536, 65544, 100003, 151936, 163848])
+def test_softmax_rows_split_over_workgroups(dev, vocab, dtype):
+    """A small batch's rows are split over workgroups: the bits of the same
+    rows in a batch that takes one workgroup per row, at one row, at an odd
+    slice count, with a tail past the last whole chunk, with masked, constant
+    and NaN rows."""
+    print(f"[case] split softmax {vocab} {dtype}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(vocab)
+    stride = (vocab + 7) // 8 * 8
+    big = (torch.randn((260, stride), device=dev, generator=g) * 3).to(dtype)[:, :vocab]
+    big[1, ::2] = float("-inf")
+    big[2, :] = 0.25
+    big[3, 17] = float("nan")
+    big[4, 5] = float("inf")
+    temps = torch.rand(260, device=dev, generator=g) + 0.3
+    temps[5] = -1.0
+    probs = torch.empty((260, stride), device=dev)[:, :vocab]
+    ref = capi.softmax_temperature(big, temps, out=probs)
+    for n in (1, 7, 31):
+        got = torch.full((n, stride), float("nan"), device=dev)[:, :vocab]
+        capi.softmax_temperature(big[:n], temps[:n], out=got)
+        torch.cuda.synchronize()
+        assert torch.equal(got.contiguous().view(torch.int32), ref[:n].contiguous().view(torch.int32))
+    if dtype == torch.float32:  # in place
+        rows = torch.empty((3, stride), device=dev)[:, :vocab].copy_(big[:3])  # aligned rows
+        capi.softmax_temperature(rows, temps[:3], out=rows)
+        torch.cuda.synchronize()
+        assert torch.equal(rows.contiguous().view(torch.int32), ref[:3].contiguous().view(torch.int32))
