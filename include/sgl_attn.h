@@ -582,6 +582,42 @@ int sgl_sampling_from_logits(const void* logits, int64_t logits_stride_row, int 
                              int32_t* out, uint8_t* success, int batch_size, int d,
                              int max_rounds, void* stream);
 
+/*
+ * Any of the draws above with a workspace: the statistics and the first sweep
+ * of a small batch's rows then run over many workgroups instead of one per
+ * row, with the same samples and success flags, bit for bit. Exactly one of
+ * probs (fp32 [batch_size, d], contiguous) and logits is given; the fields are
+ * the arguments of sgl_*_sampling_from_probs and sgl_sampling_from_logits
+ * (mode as there). workspace: sgl_sampling_workspace_bytes(batch_size, d)
+ * bytes, 16-byte aligned, written before it is read; with NULL, or where that
+ * function returns 0, each row is one workgroup's. Calls that share a
+ * workspace must be stream-ordered.
+ * Replaces: Sampler::sample's probabilities and draws (src/engine/engine.cc:306-333).
+ */
+typedef struct {
+  const float* probs;
+  const void* logits;
+  int64_t logits_stride_row;
+  const float* temperatures;
+  const float* uniform;
+  const float* top_k_f;
+  const int32_t* top_k_i;
+  const float* top_p_arr;
+  int32_t* out;
+  uint8_t* success;
+  int32_t logits_dtype;
+  int32_t mode;
+  float temperature;
+  float top_p_val;
+  int32_t top_k_val;
+  int32_t batch_size;
+  int32_t d;
+  int32_t max_rounds;
+} sgl_sampling_args_t;
+int64_t sgl_sampling_workspace_bytes(int batch_size, int d);
+int sgl_sampling_rows(const sgl_sampling_args_t* args, void* workspace, int64_t workspace_bytes,
+                      void* stream);
+
 #ifdef __cplusplus
 }  /* extern "C" */
 #endif

@@ -70,6 +70,30 @@ class PrefillPlan(ctypes.Structure):
 PREFILL_PLAN_INTS = 4096
 
 
+class SamplingArgs(ctypes.Structure):
+    """sgl_sampling_args_t."""
+    _fields_ = [
+        ("probs", ctypes.c_void_p),
+        ("logits", ctypes.c_void_p),
+        ("logits_stride_row", ctypes.c_int64),
+        ("temperatures", ctypes.c_void_p),
+        ("uniform", ctypes.c_void_p),
+        ("top_k_f", ctypes.c_void_p),
+        ("top_k_i", ctypes.c_void_p),
+        ("top_p_arr", ctypes.c_void_p),
+        ("out", ctypes.c_void_p),
+        ("success", ctypes.c_void_p),
+        ("logits_dtype", ctypes.c_int32),
+        ("mode", ctypes.c_int32),
+        ("temperature", ctypes.c_float),
+        ("top_p_val", ctypes.c_float),
+        ("top_k_val", ctypes.c_int32),
+        ("batch_size", ctypes.c_int32),
+        ("d", ctypes.c_int32),
+        ("max_rounds", ctypes.c_int32),
+    ]
+
+
 class I32Copy(ctypes.Structure):
     """sgl_i32_copy_t."""
     _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p), ("count", ctypes.c_int64)]
@@ -115,6 +139,8 @@ _SIGNATURES = {
     "sgl_silu_and_mul": ([_vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp], _i32),
     "sgl_gelu_and_mul": ([_vp, _vp, _i64, _i64, _i64, _i64, _i32, _vp], _i32),
     "sgl_softmax_temperature": ([_vp, _i64, _vp, _i64, _i32, _vp, _f32, _i64, _i64, _vp], _i32),
+    "sgl_sampling_workspace_bytes": ([_i32, _i32], _i64),
+    "sgl_sampling_rows": ([ctypes.POINTER(SamplingArgs), _vp, _i64, _vp], _i32),
     "sgl_sampling_from_logits": ([_vp, _i64, _i32, _vp, _f32, _vp, _i32, _vp, _vp, _i32, _vp, _f32,
                                   _vp, _vp, _i32, _i32, _i32, _vp], _i32),
     "sgl_sampling_from_probs": ([_vp, _vp, _vp, _i32, _i32, _i32, _vp], _i32),
@@ -721,6 +747,52 @@ def sampling_from_logits(logits: torch.Tensor, uniform_samples: torch.Tensor, mo
                                           int(top_k_val), _p(tp), float(top_p_val), _p(out),
                                           _p(succ), b, v, rounds, _stream(dev)),
            "sgl_sampling_from_logits")
+    return out, succ
+
+
+def sampling_rows(mode: str, uniform_samples: torch.Tensor, probs: Optional[torch.Tensor] = None,
+                  logits: Optional[torch.Tensor] = None,
+                  temperatures: Optional[torch.Tensor] = None, temperature: float = 1.0,
+                  top_k: Optional[torch.Tensor] = None, top_k_val: int = 0,
+                  top_p: Optional[torch.Tensor] = None, top_p_val: float = 0.0,
+                  workspace: Optional[torch.Tensor] = None):
+    """Any draw from probs or logits (exactly one) with a workspace of
+    sgl_sampling_workspace_bytes, over which a small batch's rows are split
+    (made here when none is given): the samples and flags of
+    sampling_from_logits / *_sampling_from_probs."""
+    m = {"plain": 0, "top_k": 1, "top_p": 2, "top_k_top_p": 3}[mode]
+    rows = probs if probs is not None else logits
+    dev = _need_gpu(probs, logits, uniform_samples, temperatures, top_k, top_p, workspace)
+    if probs is not None:
+        _check_probs(probs, uniform_samples, 1 if m == 0 else 2)
+    elif (logits.dim() != 2 or logits.stride(1) != 1 or uniform_samples.dtype != torch.float32
+          or not uniform_samples.is_contiguous() or uniform_samples.dim() != (1 if m == 0 else 2)
+          or uniform_samples.shape[-1] != logits.shape[0]):
+        raise ValueError("logits must be [batch, vocab] with contiguous rows and uniform_samples "
+                         "contiguous float32 [batch] or [max_rounds, batch]")
+    b, v = rows.shape
+    codes = {torch.bfloat16: SGL_DTYPE_BF16, torch.float16: SGL_DTYPE_F16,
+             torch.float32: SGL_DTYPE_F32}
+    if temperatures is not None:
+        temperatures = temperatures.to(torch.float32).reshape(b).contiguous()
+    tkf = _opt(top_k, torch.float32, b, "top_k") if m == 1 else None
+    tki = _opt(top_k, torch.int32, b, "top_k") if m == 3 else None
+    tp = _opt(top_p, torch.float32, b, "top_p") if m >= 2 else None
+    out = torch.empty(b, dtype=torch.int32, device=dev)
+    succ = None if m == 0 else torch.empty(b, dtype=torch.bool, device=dev)
+    if workspace is None:
+        workspace = torch.empty(lib().sgl_sampling_workspace_bytes(b, v), dtype=torch.uint8,
+                                device=dev)
+    args = SamplingArgs(
+        probs=_p(probs), logits=_p(logits),
+        logits_stride_row=0 if logits is None else logits.stride(0), temperatures=_p(temperatures),
+        uniform=_p(uniform_samples), top_k_f=_p(tkf), top_k_i=_p(tki), top_p_arr=_p(tp),
+        out=_p(out), success=_p(succ), logits_dtype=0 if logits is None else codes[logits.dtype],
+        mode=m, temperature=float(temperature), top_p_val=float(top_p_val),
+        top_k_val=int(top_k_val), batch_size=b, d=v,
+        max_rounds=1 if m == 0 else uniform_samples.shape[0])
+    _check(lib().sgl_sampling_rows(ctypes.byref(args), _p(workspace) if workspace.numel() else None,
+                                   workspace.numel(), _stream(dev)), "sgl_sampling_rows")
     return out, succ
 
 

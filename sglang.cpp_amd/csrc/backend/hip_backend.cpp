@@ -1000,6 +1000,30 @@ int32_t narrow_dim(int64_t v, const char* what) {
   TORCH_CHECK(v >= 0 && v <= 0x7fffffff, what, " out of range");
   return static_cast<int32_t>(v);
 }
+
+// One draw over the rows, with the workspace a small batch is split over.
+void draw_rows(const sgl_sampling_args_t& args, const torch::Tensor& rows) {
+  const int64_t bytes = sgl_sampling_workspace_bytes(args.batch_size, args.d);
+  torch::Tensor ws;
+  if (bytes > 0) ws = torch::empty({bytes}, rows.options().dtype(torch::kUInt8));
+  check_sgl(sgl_sampling_rows(&args, bytes > 0 ? ws.data_ptr() : nullptr, bytes,
+                              current_stream(rows.device())),
+            "sgl_sampling_rows");
+}
+
+sgl_sampling_args_t probs_args(const torch::Tensor& probs, const torch::Tensor& uniform, int mode,
+                               FlashInferSamplingResult& r) {
+  sgl_sampling_args_t a{};
+  a.probs = probs.data_ptr<float>();
+  a.uniform = uniform.data_ptr<float>();
+  a.mode = mode;
+  a.out = r.samples.data_ptr<int32_t>();
+  if (mode != 0) a.success = reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>());
+  a.batch_size = narrow_dim(probs.size(0), "batch");
+  a.d = narrow_dim(probs.size(1), "vocab");
+  a.max_rounds = mode == 0 ? 1 : narrow_dim(uniform.size(0), "rounds");
+  return a;
+}
 }  // namespace
 
 torch::Tensor sampling_probs(const torch::Tensor& logits, const torch::Tensor& temperatures) {
@@ -1046,31 +1070,35 @@ FlashInferSamplingResult sample_from_logits(const torch::Tensor& logits,
   FlashInferSamplingResult r;
   r.samples = torch::empty({batch}, logits.options().dtype(torch::kInt32));
   if (mode != 0) r.success = torch::empty({batch}, logits.options().dtype(torch::kBool));
-  check_sgl(sgl_sampling_from_logits(
-                logits.data_ptr(), logits.stride(0), dtype, temps.data_ptr<float>(), 1.0f,
-                uniform_samples.data_ptr<float>(), mode,
-                k_f.defined() ? k_f.data_ptr<float>() : nullptr,
-                k_i.defined() ? k_i.data_ptr<int32_t>() : nullptr, 0,
-                p_f.defined() ? p_f.data_ptr<float>() : nullptr, 0.0f, r.samples.data_ptr<int32_t>(),
-                mode != 0 ? reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>()) : nullptr,
-                narrow_dim(batch, "batch"), narrow_dim(logits.size(1), "vocab"),
-                mode == 0 ? 1 : narrow_dim(uniform_samples.size(0), "rounds"),
-                current_stream(logits.device())),
-            "sgl_sampling_from_logits");
+  sgl_sampling_args_t a{};
+  a.logits = logits.data_ptr();
+  a.logits_stride_row = logits.stride(0);
+  a.logits_dtype = dtype;
+  a.temperatures = temps.data_ptr<float>();
+  a.temperature = 1.0f;
+  a.uniform = uniform_samples.data_ptr<float>();
+  a.mode = mode;
+  a.top_k_f = k_f.defined() ? k_f.data_ptr<float>() : nullptr;
+  a.top_k_i = k_i.defined() ? k_i.data_ptr<int32_t>() : nullptr;
+  a.top_p_arr = p_f.defined() ? p_f.data_ptr<float>() : nullptr;
+  a.out = r.samples.data_ptr<int32_t>();
+  a.success = mode != 0 ? reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>()) : nullptr;
+  a.batch_size = narrow_dim(batch, "batch");
+  a.d = narrow_dim(logits.size(1), "vocab");
+  a.max_rounds = mode == 0 ? 1 : narrow_dim(uniform_samples.size(0), "rounds");
+  draw_rows(a, logits);
   return r;
 }
 
 torch::Tensor flashinfer_sample_from_probs(const torch::Tensor& probs,
-                                           const torch::Tensor& uniform_samples, bool deterministic) {
+                                           const torch::Tensor& uniform_samples,
+                                           bool /*deterministic: the sums' order is fixed*/) {
   check_probs(probs);
   check_uniform(probs, uniform_samples, 1);
-  auto samples = torch::empty({probs.size(0)}, probs.options().dtype(torch::kInt32));
-  check_sgl(sgl_sampling_from_probs(probs.data_ptr<float>(), uniform_samples.data_ptr<float>(),
-                                    samples.data_ptr<int32_t>(), narrow_dim(probs.size(0), "batch"),
-                                    narrow_dim(probs.size(1), "vocab"), deterministic ? 1 : 0,
-                                    current_stream(probs.device())),
-            "sgl_sampling_from_probs");
-  return samples;
+  FlashInferSamplingResult r;
+  r.samples = torch::empty({probs.size(0)}, probs.options().dtype(torch::kInt32));
+  draw_rows(probs_args(probs, uniform_samples, 0, r), probs);
+  return r.samples;
 }
 
 FlashInferSamplingResult flashinfer_top_k_sample_from_probs(const torch::Tensor& probs,
@@ -1081,14 +1109,10 @@ FlashInferSamplingResult flashinfer_top_k_sample_from_probs(const torch::Tensor&
   check_uniform(probs, uniform_samples, 2);
   check_row_arg(top_k, probs, torch::kFloat32, "top_k");
   auto r = sampling_outputs(probs);
-  check_sgl(sgl_top_k_sampling_from_probs(
-                probs.data_ptr<float>(), uniform_samples.data_ptr<float>(), r.samples.data_ptr<int32_t>(),
-                reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>()),
-                top_k.defined() ? top_k.data_ptr<float>() : nullptr,
-                narrow_dim(probs.size(0), "batch"), static_cast<int>(top_k_value),
-                narrow_dim(probs.size(1), "vocab"), narrow_dim(uniform_samples.size(0), "rounds"),
-                deterministic ? 1 : 0, current_stream(probs.device())),
-            "sgl_top_k_sampling_from_probs");
+  auto a = probs_args(probs, uniform_samples, 1, r);
+  a.top_k_f = top_k.defined() ? top_k.data_ptr<float>() : nullptr;
+  a.top_k_val = static_cast<int>(top_k_value);
+  draw_rows(a, probs);
   return r;
 }
 
@@ -1100,14 +1124,10 @@ FlashInferSamplingResult flashinfer_top_p_sample_from_probs(const torch::Tensor&
   check_uniform(probs, uniform_samples, 2);
   check_row_arg(top_p, probs, torch::kFloat32, "top_p");
   auto r = sampling_outputs(probs);
-  check_sgl(sgl_top_p_sampling_from_probs(
-                probs.data_ptr<float>(), uniform_samples.data_ptr<float>(), r.samples.data_ptr<int32_t>(),
-                reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>()),
-                top_p.defined() ? top_p.data_ptr<float>() : nullptr,
-                narrow_dim(probs.size(0), "batch"), static_cast<float>(top_p_value),
-                narrow_dim(probs.size(1), "vocab"), narrow_dim(uniform_samples.size(0), "rounds"),
-                deterministic ? 1 : 0, current_stream(probs.device())),
-            "sgl_top_p_sampling_from_probs");
+  auto a = probs_args(probs, uniform_samples, 2, r);
+  a.top_p_arr = top_p.defined() ? top_p.data_ptr<float>() : nullptr;
+  a.top_p_val = static_cast<float>(top_p_value);
+  draw_rows(a, probs);
   return r;
 }
 
@@ -1119,16 +1139,12 @@ FlashInferSamplingResult flashinfer_top_k_top_p_sample_from_probs(
   check_row_arg(top_k, probs, torch::kInt32, "top_k");
   check_row_arg(top_p, probs, torch::kFloat32, "top_p");
   auto r = sampling_outputs(probs);
-  check_sgl(sgl_top_k_top_p_sampling_from_probs(
-                probs.data_ptr<float>(), uniform_samples.data_ptr<float>(),
-                top_k.defined() ? top_k.data_ptr<int32_t>() : nullptr,
-                top_p.defined() ? top_p.data_ptr<float>() : nullptr, r.samples.data_ptr<int32_t>(),
-                reinterpret_cast<uint8_t*>(r.success.data_ptr<bool>()),
-                narrow_dim(probs.size(0), "batch"), static_cast<int>(top_k_value),
-                static_cast<float>(top_p_value), narrow_dim(probs.size(1), "vocab"),
-                narrow_dim(uniform_samples.size(0), "rounds"), deterministic ? 1 : 0,
-                current_stream(probs.device())),
-            "sgl_top_k_top_p_sampling_from_probs");
+  auto a = probs_args(probs, uniform_samples, 3, r);
+  a.top_k_i = top_k.defined() ? top_k.data_ptr<int32_t>() : nullptr;
+  a.top_k_val = static_cast<int>(top_k_value);
+  a.top_p_arr = top_p.defined() ? top_p.data_ptr<float>() : nullptr;
+  a.top_p_val = static_cast<float>(top_p_value);
+  draw_rows(a, probs);
   return r;
 }
 

@@ -536,18 +536,23 @@ struct HeldSweep {
   }
 };
 
-template <class Src, class Sweep>
+// The first sweep already copies the probabilities above this: at most
+// 1 / kCandThr of them in a normalised row, so any pivot at or above it is
+// served from LDS.
+constexpr float kCandThr = 1.f / static_cast<float>(kCandCap - kCandCap / 8);
+
+// The row's draws. kPre: the block masses of the first sweep and, where they
+// fit (pre_cand), its copies are in sh already, its mass and count are not.
+template <bool kPre, class Src, class Sweep>
 __device__ __forceinline__ void sample_row(const SampleArgs& a, const Src& row, const Sweep& rs,
-                                           Shared& sh) {
+                                           Shared& sh, bool pre_cand = false) {
   const int row_id = blockIdx.x;
   const bool cand_ok = a.mode != 0 && (a.d + kBlock - 1) / kBlock <= kCandBlocks;
-  // The first sweep already copies the probabilities above cand_thr: at
-  // most 1 / cand_thr of them in a normalised row, so any pivot at or above
-  // cand_thr is served from LDS.
-  float cand_thr = 1.f / static_cast<float>(kCandCap - kCandCap / 8);
-  bool cand = false;  // the copies hold every probability above cand_thr
+  float cand_thr = kCandThr;
+  bool cand = pre_cand;  // the copies hold every probability above cand_thr
   float u = a.uniform[row_id];
-  if (cand_ok) {
+  if (kPre) {
+  } else if (cand_ok) {
     if (threadIdx.x == 0) sh.ncand = 0;
     rs.template run<true>(0.f, cand_thr, sh);
     cand = sh.ncand <= kCandCap;
@@ -588,6 +593,8 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const Src& row, 
       } else {
         rs.template run<false>(pivot, 0.f, sh);
       }
+    } else if (kPre && pivot == 0.f) {
+      rs.template run<false>(0.f, 0.f, sh);  // nothing drawn: the first sweep's mass and count
     }
     q = sh.total;
     const int count = sh.count;
@@ -612,7 +619,7 @@ __global__ void __launch_bounds__(kThreads) sampling_kernel(SampleArgs a) {
   const int row_id = blockIdx.x;
   if constexpr (SRC < 0) {
     const ProbRow row{a.probs + static_cast<int64_t>(row_id) * a.d};
-    sample_row(a, row, StreamSweep<ProbRow>{row, a.d, a.vec}, sh);
+    sample_row<false>(a, row, StreamSweep<ProbRow>{row, a.d, a.vec}, sh);
   } else {
     static_assert(kThreads == sp::kStatLanes, "one statistics lane per thread");
     constexpr int B = 16 / sp::Elem<SRC>::kPer;
@@ -623,7 +630,7 @@ __global__ void __launch_bounds__(kThreads) sampling_kernel(SampleArgs a) {
     const float m = sp::block_max<kWaves>(st.mx, sh.wave_f);
     const float inv_s = 1.0f / sp::block_sum<kWaves>(sp::lane_sum_at(st, m, sc), sh.wave_f);
     const LogitRow<SRC> row{x, sc, sp::exp2_offset(m, sc), inv_s};
-    sample_row(a, row, StreamSweep<LogitRow<SRC>>{row, a.d, a.vec}, sh);
+    sample_row<false>(a, row, StreamSweep<LogitRow<SRC>>{row, a.d, a.vec}, sh);
   }
 }
 
@@ -665,7 +672,7 @@ __global__ void __launch_bounds__(kThreads) sampling_held_kernel(SampleArgs a) {
 #pragma unroll
   for (int k = 0; k < NC; ++k) asm volatile("" : "+v"(held[k]));
   const LogitRow<SRC> row{x, sc, nb, inv_s};
-  sample_row(a, row, HeldSweep<SRC, NC>{held, row, a.d, sc, nb, inv_s}, sh);
+  sample_row<false>(a, row, HeldSweep<SRC, NC>{held, row, a.d, sc, nb, inv_s}, sh);
 }
 
 template <int SRC>
@@ -684,13 +691,227 @@ void launch_held(const SampleArgs& a, int per_lane, dim3 grid, dim3 block, hipSt
     hipLaunchKernelGGL((sampling_held_kernel<SRC, kMaxHeldChunks>), grid, block, 0, s, a);
 }
 
-int launch_sampling(const SampleArgs& a, void* stream) {
+// ------------------------------------------------------------------ rows over workgroups
+//
+// With one workgroup per row a small batch leaves most CUs idle while each
+// row's statistics and first sweep (the two passes over the whole row) run on
+// one. With a workspace these passes are launches of their own over slices of
+// the rows, in the same lanes, blocks and orders, so the draws keep their
+// bits; the rounds stay with one workgroup per row, which starts from the
+// block masses and copies it finds in the workspace.
+//
+// A row's workspace: the 1024 statistics lanes (draws from logits), the block
+// masses, the blocks' copy counts, and each block's copies at 512 times its
+// index.
+struct SplitLayout {
+  int64_t mass, count, copies, row;  // byte offsets, bytes per row
+};
+__device__ __host__ inline SplitLayout split_layout(int d) {
+  const int64_t nblk = (static_cast<int64_t>(d) + kBlock - 1) / kBlock, pad = (nblk + 63) / 64 * 64;
+  SplitLayout l;
+  l.mass = sp::kStatLanes * 8;
+  l.count = l.mass + pad * 4;
+  l.copies = l.count + pad * 4;
+  l.row = l.copies + nblk * kBlock * 4;
+  return l;
+}
+
+// One wave per 64 statistics lanes.
+template <int DT>
+__global__ void __launch_bounds__(kWave) sampling_lane_stats(SampleArgs a, char* ws) {
+  constexpr int B = 16 / sp::Elem<DT>::kPer;
+  const int r = blockIdx.y;
+  const char* x = static_cast<const char*>(a.logits) + static_cast<int64_t>(r) * a.x_st * B;
+  const int v = blockIdx.x * kWave + threadIdx.x;
+  const float sc = sp::exp2_scale(a.temps ? a.temps[r] : a.temp);
+  const sp::LaneStats st = sp::lane_stats<DT>(x, a.d, a.stats_vec, v, sc);
+  reinterpret_cast<float2*>(ws + r * split_layout(a.d).row)[v] = float2{st.mx, st.s};
+}
+
+// Row source of a split launch: the fp32 probabilities, or the logits with the
+// row constants folded from the lanes' states (the whole workgroup).
+template <int SRC>
+__device__ __forceinline__ auto split_source(const SampleArgs& a, const char* wrow, int r, float* red) {
+  if constexpr (SRC < 0) {
+    return ProbRow{a.probs + static_cast<int64_t>(r) * a.d};
+  } else {
+    constexpr int B = 16 / sp::Elem<SRC>::kPer;
+    const float2 lane = reinterpret_cast<const float2*>(wrow)[threadIdx.x];
+    const float sc = sp::exp2_scale(a.temps ? a.temps[r] : a.temp);
+    sp::LaneStats st;
+    st.mx = lane.x;
+    st.s = lane.y;
+    const float m = sp::block_max<kWaves>(st.mx, red);
+    const float inv_s = 1.0f / sp::block_sum<kWaves>(sp::lane_sum_at(st, m, sc), red);
+    return LogitRow<SRC>{static_cast<const char*>(a.logits) + static_cast<int64_t>(r) * a.x_st * B,
+                         sc, sp::exp2_offset(m, sc), inv_s};
+  }
+}
+
+// The first sweep: one block of 512 probabilities per wave, its mass and its
+// copies as sweep_block makes them.
+template <int SRC>
+__global__ void __launch_bounds__(kThreads) sampling_first_sweep(SampleArgs a, char* ws) {
+  __shared__ float red[kWaves];
+  const int r = blockIdx.y;
+  const SplitLayout l = split_layout(a.d);
+  char* wrow = ws + r * l.row;
+  const auto row = split_source<SRC>(a, wrow, r, red);
+  const int lane = threadIdx.x & 63;
+  const int b = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (b * kBlock >= a.d) return;
+  BlockVals bv;
+  load_block(row, b, a.d, a.vec && (b + 1) * kBlock <= a.d, bv);
+  float m = 0.f;
+#pragma unroll
+  for (int s = 0; s < kSub; ++s)
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) m += bv.v[s][j] > 0.f ? bv.v[s][j] : 0.f;
+  m = wave_sum_f(m);
+  if (lane == 0) reinterpret_cast<float*>(wrow + l.mass)[b] = m;
+  if (a.mode == 0) return;
+  float* copies = reinterpret_cast<float*>(wrow + l.copies) + static_cast<int64_t>(b) * kBlock;
+  int pos = 0;
+#pragma unroll
+  for (int s = 0; s < kSub; ++s)
+#pragma unroll
+    for (int j = 0; j < kVec; ++j) {
+      const float x = bv.v[s][j];
+      const uint64_t mj = __ballot(x > kCandThr);
+      if (mj != 0) {
+        if (x > kCandThr) copies[pos + lanes_below(mj)] = x;
+        pos += __builtin_popcountll(mj);
+      }
+    }
+  if (lane == 0) reinterpret_cast<int*>(wrow + l.count)[b] = pos;
+}
+
+// The rounds, one workgroup per row. The masses, the counts and the first 16
+// copies of every block are one trip to memory.
+template <int SRC>
+__global__ void __launch_bounds__(kThreads) sampling_split_rounds(SampleArgs a, const char* ws) {
+  __shared__ Shared sh;
+  const int r = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const SplitLayout l = split_layout(a.d);
+  const char* wrow = ws + r * l.row;
+  const int nblk = (a.d + kBlock - 1) / kBlock;
+  const float* mass = reinterpret_cast<const float*>(wrow + l.mass);
+  const int* count = reinterpret_cast<const int*>(wrow + l.count);
+  const float* copies = reinterpret_cast<const float*>(wrow + l.copies);
+  // Blocks 2 tid and 2 tid + 1 (nblk <= kCandBlocks = 2 kThreads).
+  int n0 = 0, n1 = 0;
+  float m0 = 0.f, m1 = 0.f;
+  if (2 * tid < nblk) m0 = mass[2 * tid];
+  if (2 * tid + 1 < nblk) m1 = mass[2 * tid + 1];
+  if (a.mode != 0) {
+    if (2 * tid < nblk) n0 = count[2 * tid];
+    if (2 * tid + 1 < nblk) n1 = count[2 * tid + 1];
+  }
+  // A group of 16 lanes copies blocks 4 wave + lane / 16 + 64 k; most have at
+  // most 16 copies.
+  constexpr int kAhead = 8;
+  const int sub = lane & 15, g0 = 4 * wave + (lane >> 4);
+  float head[kAhead];
+  if (a.mode != 0) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int b = g0 + 64 * k;
+      head[k] = b < nblk ? copies[static_cast<int64_t>(b) * kBlock + sub] : 0.f;
+    }
+  }
+  const auto row = split_source<SRC>(a, wrow, r, sh.wave_f);
+  if (2 * tid < nblk) sh.pool[2 * tid] = m0;
+  if (2 * tid + 1 < nblk) sh.pool[2 * tid + 1] = m1;
+  bool cand = false;
+  if (a.mode != 0) {
+    // Where each block's copies start: a scan of the counts (exact in fp32).
+    const float own = static_cast<float>(n0 + n1);
+    const float incl = wave_scan(own);
+    if (lane == kWave - 1) sh.wave_n[wave] = incl;
+    __syncthreads();
+    float before = 0.f, total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      before += w < wave ? sh.wave_n[w] : 0.f;
+      total += sh.wave_n[w];
+    }
+    cand = total <= static_cast<float>(kCandCap);
+    if (cand) {
+      const int start = static_cast<int>(before + incl - own);
+      if (2 * tid < nblk) sh.seg[2 * tid] = static_cast<uint32_t>(start) | static_cast<uint32_t>(n0) << 16;
+      if (2 * tid + 1 < nblk)
+        sh.seg[2 * tid + 1] = static_cast<uint32_t>(start + n0) | static_cast<uint32_t>(n1) << 16;
+      __syncthreads();
+      auto place = [&](int b, float first) {
+        const uint32_t sg = sh.seg[b];
+        const int at = kCandBlocks + static_cast<int>(sg & 0xFFFF), n = static_cast<int>(sg >> 16);
+        if (sub < n) sh.pool[at + sub] = first;
+        for (int i = sub + 16; i < n; i += 16)
+          sh.pool[at + i] = copies[static_cast<int64_t>(b) * kBlock + i];
+      };
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k)
+        if (g0 + 64 * k < nblk) place(g0 + 64 * k, head[k]);
+      for (int b = g0 + 64 * kAhead; b < nblk; b += 64)
+        place(b, copies[static_cast<int64_t>(b) * kBlock + sub]);
+    }
+  }
+  __syncthreads();
+  using Src = std::remove_const_t<decltype(row)>;
+  sample_row<true>(a, row, StreamSweep<Src>{row, a.d, a.vec}, sh, cand);
+}
+
+// Bytes of a split batch's workspace, 0 where one workgroup per row is the
+// better: rows long enough for the extra launches, batches that leave CUs
+// idle. Top-k + top-p, us, one workgroup per row -> split, from probabilities
+// and from bf16 logits: 151,936 x 1 24.0 -> 12.6, 34.2 -> 18.5; x 16 38.6 -> 28.5,
+// 54.8 -> 41.3; x 64 44.7 -> 38.6, 66.3 -> 60.7; x 128 47.1 against 47.4, 68.0
+// against 73.4; 65,536 x 32 22.5 -> 21.2, 29.2 -> 28.2; x 48 22.5 -> 21.9, 30.1
+// against 30.7. What is left is the slowest row's rounds and repeated sweeps,
+// one workgroup's at about 3 and 8 to 10 us each.
+int64_t split_workspace(int64_t batch, int64_t d) {
+  if (batch <= 0 || d < 65536 || d > static_cast<int64_t>(kCandBlocks) * kBlock || batch * 2000 > d)
+    return 0;
+  return batch * split_layout(static_cast<int>(d)).row;
+}
+
+template <int SRC>
+int launch_split(const SampleArgs& a, char* ws, hipStream_t s) {
+  if constexpr (SRC >= 0) {
+    hipLaunchKernelGGL((sampling_lane_stats<SRC>), dim3(sp::kStatWaves, a.batch), dim3(kWave), 0, s,
+                       a, ws);
+    const int st = launch_status();
+    if (st != SGL_OK) return st;
+  }
+  const int nblk = (a.d + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL((sampling_first_sweep<SRC>), dim3((nblk + kWaves - 1) / kWaves, a.batch),
+                     dim3(kThreads), 0, s, a, ws);
+  const int st = launch_status();
+  if (st != SGL_OK) return st;
+  hipLaunchKernelGGL((sampling_split_rounds<SRC>), dim3(a.batch), dim3(kThreads), 0, s, a, ws);
+  return launch_status();
+}
+
+// A workspace (split_workspace bytes) splits the rows; without one, or for a
+// batch that is not split, each row is one workgroup's.
+int launch_sampling(const SampleArgs& a, void* stream, void* ws = nullptr, int64_t ws_bytes = 0) {
   if (a.batch < 0 || a.d <= 0 || (a.mode != 0 && a.rounds <= 0)) return SGL_ERR_INVALID_ARG;
   if ((static_cast<int64_t>(a.d) + kBlock - 1) / kBlock > kMaxBlocks) return SGL_ERR_UNSUPPORTED;
   if (a.batch == 0) return SGL_OK;
   if (!a.uniform || !a.out) return SGL_ERR_INVALID_ARG;
   const dim3 grid(a.batch), block(kThreads);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const int64_t need = split_workspace(a.batch, a.d);
+  if (ws && need > 0 && (a.probs || a.logits)) {
+    if (ws_bytes < need) return SGL_ERR_CAPACITY;
+    if (!aligned16(ws)) return SGL_ERR_ALIGNMENT;
+    char* w = static_cast<char*>(ws);
+    if (a.probs) return launch_split<-1>(a, w, s);
+    if (a.logit_dtype == SGL_DTYPE_BF16) return launch_split<SGL_DTYPE_BF16>(a, w, s);
+    if (a.logit_dtype == SGL_DTYPE_F16) return launch_split<SGL_DTYPE_F16>(a, w, s);
+    return launch_split<SGL_DTYPE_F32>(a, w, s);
+  }
   if (a.probs) {
     hipLaunchKernelGGL(sampling_kernel<-1>, grid, block, 0, s, a);
   } else if (a.logits) {
@@ -776,21 +997,24 @@ extern "C" int sgl_top_k_top_p_sampling_from_probs(const float* probs, const flo
   return launch_sampling(a, stream);
 }
 
-extern "C" int sgl_sampling_from_logits(const void* logits, int64_t logits_stride_row,
-                                        int logits_dtype, const float* temperatures,
-                                        float temperature, const float* uniform, int mode,
-                                        const float* top_k_f, const int32_t* top_k_i,
-                                        int top_k_val, const float* top_p_arr, float top_p_val,
-                                        int32_t* out, uint8_t* success, int batch_size, int d,
-                                        int max_rounds, void* stream) {
+// Checks and arguments of a draw from logits; *done when there is nothing to do.
+static int logits_args(const void* logits, int64_t logits_stride_row, int logits_dtype,
+                       const float* temperatures, float temperature, const float* uniform, int mode,
+                       const float* top_k_f, const int32_t* top_k_i, int top_k_val,
+                       const float* top_p_arr, float top_p_val, int32_t* out, uint8_t* success,
+                       int batch_size, int d, int max_rounds, SampleArgs& a, bool& done) {
+  done = false;
   if (mode < 0 || mode > 3 || d <= 0 || logits_stride_row < d) return SGL_ERR_INVALID_ARG;
-  if (batch_size == 0) return SGL_OK;
+  if (batch_size == 0) {
+    done = true;
+    return SGL_OK;
+  }
   if (!logits || (!temperatures && !(temperature > 0.f))) return SGL_ERR_INVALID_ARG;
   int esize;
   if (logits_dtype == SGL_DTYPE_BF16 || logits_dtype == SGL_DTYPE_F16) esize = 2;
   else if (logits_dtype == SGL_DTYPE_F32) esize = 4;
   else return SGL_ERR_UNSUPPORTED;
-  SampleArgs a = base_args(nullptr, uniform, out, mode == 0 ? nullptr : success, batch_size, d,
+  a = base_args(nullptr, uniform, out, mode == 0 ? nullptr : success, batch_size, d,
                            mode == 0 ? 1 : max_rounds, mode);
   a.logits = logits;
   a.x_st = logits_stride_row;
@@ -806,5 +1030,51 @@ extern "C" int sgl_sampling_from_logits(const void* logits, int64_t logits_strid
     a.top_p_arr = top_p_arr;
     a.top_p_val = top_p_val;
   }
-  return launch_sampling(a, stream);
+  return SGL_OK;
+}
+
+extern "C" int sgl_sampling_from_logits(const void* logits, int64_t logits_stride_row,
+                                        int logits_dtype, const float* temperatures,
+                                        float temperature, const float* uniform, int mode,
+                                        const float* top_k_f, const int32_t* top_k_i,
+                                        int top_k_val, const float* top_p_arr, float top_p_val,
+                                        int32_t* out, uint8_t* success, int batch_size, int d,
+                                        int max_rounds, void* stream) {
+  SampleArgs a;
+  bool done;
+  const int st = logits_args(logits, logits_stride_row, logits_dtype, temperatures, temperature,
+                             uniform, mode, top_k_f, top_k_i, top_k_val, top_p_arr, top_p_val, out,
+                             success, batch_size, d, max_rounds, a, done);
+  return st != SGL_OK || done ? st : launch_sampling(a, stream);
+}
+
+extern "C" int64_t sgl_sampling_workspace_bytes(int batch_size, int d) {
+  return split_workspace(batch_size, d);
+}
+
+extern "C" int sgl_sampling_rows(const sgl_sampling_args_t* in, void* workspace,
+                                 int64_t workspace_bytes, void* stream) {
+  if (!in || (in->probs && in->logits)) return SGL_ERR_INVALID_ARG;
+  SampleArgs a;
+  if (in->probs) {
+    if (in->mode < 0 || in->mode > 3) return SGL_ERR_INVALID_ARG;
+    a = base_args(in->probs, in->uniform, in->out, in->mode == 0 ? nullptr : in->success,
+                  in->batch_size, in->d, in->mode == 0 ? 1 : in->max_rounds, in->mode);
+    if (in->mode == 1) a.top_k_f = in->top_k_f;
+    if (in->mode == 3) a.top_k_i = in->top_k_i;
+    a.top_k_val = in->top_k_val;
+    if (in->mode >= 2) {
+      a.top_p_arr = in->top_p_arr;
+      a.top_p_val = in->top_p_val;
+    }
+  } else {
+    bool done;
+    const int st = logits_args(in->logits, in->logits_stride_row, in->logits_dtype,
+                               in->temperatures, in->temperature, in->uniform, in->mode,
+                               in->top_k_f, in->top_k_i, in->top_k_val, in->top_p_arr,
+                               in->top_p_val, in->out, in->success, in->batch_size, in->d,
+                               in->max_rounds, a, done);
+    if (st != SGL_OK || done) return st;
+  }
+  return launch_sampling(a, stream, workspace, workspace_bytes);
 }

@@ -541,3 +541,44 @@ def test_softmax_rows_split_over_workgroups(dev, vocab, dtype):
         capi.softmax_temperature(rows, temps[:3], out=rows)
         torch.cuda.synchronize()
         assert torch.equal(rows.contiguous().view(torch.int32), ref[:3].contiguous().view(torch.int32))
+
+
+@pytest.mark.parametrize("source", ["probs", torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("vocab", [65536, 65543, 66048 + 8, 151936, 200008, 1 << 20])
+def test_rows_split_over_workgroups_draw_the_same(dev, vocab, source):
+    """A small batch's rows split over workgroups (a workspace of any content)
+    give the samples and flags of one workgroup per row: all four draws, odd
+    lengths, flat rows (repeated sweeps, copies that overflow), peaked,
+    constant, masked and NaN rows."""
+    note(f"split draws {vocab} {source}")
+    n = min(13, vocab // 2000)
+    g = torch.Generator(device=dev).manual_seed(vocab)
+    x = torch.randn((n, vocab), device=dev, generator=g) * torch.linspace(0.2, 6, n, device=dev)[:, None]
+    x[1, ::3] = float("-inf")
+    x[2] = 0.5
+    x[3, vocab // 2] = 60.0
+    temps = torch.rand(n, device=dev, generator=g) + 0.5
+    temps[4] = -1.0  # a NaN row
+    k = torch.randint(1, 300, (n,), device=dev, generator=g)
+    p = torch.rand(n, device=dev, generator=g)
+    none = torch.empty(0, dtype=torch.uint8, device=dev)
+    ws = torch.full((capi.lib().sgl_sampling_workspace_bytes(n, vocab),), 255, dtype=torch.uint8,
+                    device=dev)
+    assert ws.numel() > 0
+    if source == "probs":
+        rows = dict(probs=torch.softmax(x / temps[:, None], -1).contiguous())
+        rows["probs"][4] = float("nan")
+        rows["probs"][5] = 0.0
+    else:
+        rows = dict(logits=x.to(source), temperatures=temps)
+    for mode in ("plain", "top_k", "top_p", "top_k_top_p"):
+        u = torch.rand((n,) if mode == "plain" else (6, n), device=dev, generator=g)
+        args = dict(rows, top_k=k.to(torch.float32 if mode == "top_k" else torch.int32)
+                    if "top_k" in mode else None, top_p=p if "top_p" in mode else None)
+        one = capi.sampling_rows(mode, u, workspace=none, **args)
+        two = capi.sampling_rows(mode, u, workspace=ws, **args)
+        torch.cuda.synchronize()
+        assert torch.equal(one[0], two[0]), mode
+        assert mode == "plain" or torch.equal(one[1], two[1]), mode
+    with pytest.raises(capi.SglError):
+        capi.sampling_rows("plain", torch.rand(n, device=dev), workspace=ws[:-64], **rows)
