@@ -326,6 +326,25 @@ int sgl_paged_decode_noalloc(const sgl_decode_plan_t* plan, const void* q,
 #define SGL_DECODE_SCRATCH_BYTES (32ll << 20)
 
 /*
+ * The attention layer's decode step: sgl_fused_qknorm_rope_store (with
+ * SGL_FUSED_NO_K_WRITEBACK) on the batch's tokens, token r of qkv being request
+ * r's, then sgl_paged_decode of the rotated q rows over the pool (k_cache and
+ * v_cache [slots, Hkv, D] contiguous), with the same results. Batches of at
+ * most 64 requests that sgl_paged_decode takes in one kernel run as one launch
+ * here too; others as those two calls.
+ * Replaces: AttentionLayer::forward's norm, RoPE, store and decode
+ *           (src/layers/attention_layer.cc:27-47, src/attention/flashinfer_backend.cu:530-595).
+ */
+int sgl_decode_layer(const sgl_decode_plan_t* plan, void* qkv, int64_t qkv_stride_token,
+                     void* k_cache, void* v_cache, const void* q_weight, const void* k_weight,
+                     const float* cos_cache, const float* sin_cache, const int32_t* positions,
+                     const int32_t* out_loc, float eps, const int32_t* indices,
+                     const int32_t* kv_indptr, int batch_size, int num_qo_heads,
+                     int num_kv_heads, int head_dim, float sm_scale, void* o,
+                     int64_t o_stride_token, int64_t o_stride_head, void* workspace,
+                     int64_t workspace_bytes, void* stream);
+
+/*
  * Reads the status word a decode call left in its workspace (waits for the
  * stream): SGL_OK, or SGL_ERR_CAPACITY when the batch exceeded its plan.
  * workspace NULL reads the word of sgl_paged_decode_noalloc's scratch on the

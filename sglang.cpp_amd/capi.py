@@ -150,6 +150,9 @@ _SIGNATURES = {
                                        _vp], _i32),
     "sgl_top_k_top_p_sampling_from_probs": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _i32,
                                              _i32, _i32, _vp], _i32),
+    "sgl_decode_layer": ([ctypes.POINTER(DecodePlan), _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                          _vp, _f32, _vp, _vp, _i32, _i32, _i32, _i32, _f32, _vp, _i64, _i64, _vp,
+                          _i64, _vp], _i32),
     "sgl_paged_prefill": ([_vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp, _vp, _vp, _vp, _i32,
                            _i32, _i32, _i32, _i32, _f32, _vp, _i64, _i64, _vp], _i32),
     "sgl_prefill_plan": ([_vp, _vp, _i32, _i32, _i32, _i32, ctypes.POINTER(PrefillPlan), _vp,
@@ -548,6 +551,30 @@ def decode_plan_check(plan: DecodePlan, kv_indptr_host: Sequence[int]) -> int:
 def decode_workspace(plan: DecodePlan, device: torch.device) -> torch.Tensor:
     """Allocates the split-KV workspace a plan needs."""
     return torch.empty(int(plan.workspace_bytes), dtype=torch.uint8, device=device)
+
+
+def decode_layer(plan: DecodePlan, qkv: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
+                 q_weight: Optional[torch.Tensor], k_weight: Optional[torch.Tensor],
+                 cos: torch.Tensor, sin: torch.Tensor, positions: torch.Tensor,
+                 out_loc: torch.Tensor, eps: float, indices: torch.Tensor, kv_indptr: torch.Tensor,
+                 num_qo_heads: int, o: torch.Tensor, workspace: torch.Tensor,
+                 sm_scale: Optional[float] = None) -> None:
+    """sgl_decode_layer: norm, RoPE, store and decode of the batch's tokens
+    (qkv [batch, (Hq + 2 Hkv) D], the q part rotated in place; o [batch, Hq, D])."""
+    dev = _need_gpu(qkv, k_cache, v_cache, q_weight, k_weight, cos, sin, positions, out_loc, indices,
+                    kv_indptr, o, workspace)
+    if not (k_cache.is_contiguous() and v_cache.is_contiguous()) or qkv.stride(1) != 1:
+        raise ValueError("the caches must be contiguous and qkv's rows too")
+    if any(t.dtype != torch.int32 for t in (positions, out_loc, indices, kv_indptr)):
+        raise ValueError("positions, out_loc, indices and kv_indptr must be int32")
+    hkv, D = k_cache.shape[1], k_cache.shape[2]
+    scale = 1.0 / math.sqrt(D) if sm_scale is None else sm_scale
+    _check(lib().sgl_decode_layer(
+        ctypes.byref(plan), _p(qkv), qkv.stride(0), _p(k_cache), _p(v_cache), _p(q_weight),
+        _p(k_weight), _p(cos), _p(sin), _p(positions), _p(out_loc), float(eps), _p(indices),
+        _p(kv_indptr), kv_indptr.shape[0] - 1, num_qo_heads, hkv, D, scale, _p(o), o.stride(0),
+        o.stride(1), _p(workspace), workspace.numel() * workspace.element_size(), _stream(dev)),
+        "sgl_decode_layer")
 
 
 def decode_status(workspace: Optional[torch.Tensor]) -> int:

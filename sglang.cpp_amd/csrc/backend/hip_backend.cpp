@@ -389,6 +389,51 @@ torch::Tensor HipAttnBackend::forward(const torch::Tensor& q, const torch::Tenso
   return attend(q.view({-1, num_qo_heads_, head_dim_}), layer_id, batch);
 }
 
+torch::Tensor& HipAttnBackend::decode_workspace(const HipAttnMetadata& meta, void* stream) {
+  // Graph-captured launches use the capture workspace, whose address never
+  // changes; eager launches use the growable one, which is kept alive if a
+  // graph records it anyway (capture of eagerly prepared metadata).
+  torch::Tensor& ws = !meta.use_capture_buffers ? workspace(meta.dec_plan.workspace_bytes)
+                      : meta.is_prefill         ? mixed_->workspace
+                                                : capture_->workspace;
+  if (!meta.use_capture_buffers) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    check_hip(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cs), "hipStreamIsCapturing");
+    if (cs != hipStreamCaptureStatusNone) workspace_captured_ = true;
+  }
+  TORCH_CHECK(ws.numel() >= meta.dec_plan.workspace_bytes, "decode workspace too small");
+  return ws;
+}
+
+bool HipAttnBackend::decode_layer_fits(const torch::Tensor& qkv, Batch& batch) const {
+  auto meta = metadata_of(batch);
+  return !meta->is_prefill && meta->num_prefill == 0 && meta->num_decode > 0 &&
+         meta->num_decode == qkv.size(0);
+}
+
+torch::Tensor HipAttnBackend::decode_layer(const torch::Tensor& qkv, const torch::Tensor& positions,
+                                           const void* q_weight, const void* k_weight, float eps,
+                                           const torch::Tensor& cos, const torch::Tensor& sin,
+                                           int layer_id, Batch& batch) {
+  auto meta = metadata_of(batch);
+  auto o = torch::empty({qkv.size(0), num_qo_heads_, head_dim_}, qkv.options());
+  auto kc = kv_cache_->k_cache(layer_id);
+  auto vc = kv_cache_->v_cache(layer_id);
+  void* stream = current_stream(kv_cache_->device());
+  torch::Tensor& ws = decode_workspace(*meta, stream);
+  check_sgl(sgl_decode_layer(&meta->dec_plan, qkv.data_ptr(), qkv.stride(0), kc.data_ptr(),
+                             vc.data_ptr(), q_weight, k_weight, cos.data_ptr<float>(),
+                             sin.data_ptr<float>(), positions.data_ptr<int32_t>(),
+                             batch.out_loc.data_ptr<int32_t>(), eps,
+                             meta->dec_indices.data_ptr<int32_t>(),
+                             meta->dec_kv_indptr.data_ptr<int32_t>(), meta->num_decode,
+                             num_qo_heads_, num_kv_heads_, head_dim_,
+                             1.0f / std::sqrt(static_cast<float>(head_dim_)), o.data_ptr(),
+                             o.stride(0), o.stride(1), ws.data_ptr(), ws.numel(), stream),
+            "sgl_decode_layer");
+  return o.view({-1, num_qo_heads_ * head_dim_});
+}
+
 torch::Tensor HipAttnBackend::attend(const torch::Tensor& q_in, int layer_id, Batch& batch) {
   auto meta = metadata_of(batch);
   auto q = q_in.dim() == 2 ? q_in.view({-1, num_qo_heads_, head_dim_}) : q_in;
@@ -442,19 +487,7 @@ torch::Tensor HipAttnBackend::attend(const torch::Tensor& q_in, int layer_id, Ba
               "hipStreamWaitEvent");
   }
   if (meta->num_decode > 0) {
-    // Graph-captured launches use the capture workspace, whose address never
-    // changes; eager launches use the growable one, which is kept alive if a
-    // graph records it anyway (capture of eagerly prepared metadata).
-    torch::Tensor& ws = !meta->use_capture_buffers ? workspace(meta->dec_plan.workspace_bytes)
-                        : meta->is_prefill         ? mixed_->workspace
-                                                   : capture_->workspace;
-    if (!meta->use_capture_buffers) {
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      check_hip(hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cs),
-                "hipStreamIsCapturing");
-      if (cs != hipStreamCaptureStatusNone) workspace_captured_ = true;
-    }
-    TORCH_CHECK(ws.numel() >= meta->dec_plan.workspace_bytes, "decode workspace too small");
+    torch::Tensor& ws = decode_workspace(*meta, stream);
     check_sgl(sgl_paged_decode(&meta->dec_plan, q.data_ptr(), q.stride(0), q.stride(1),
                                kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1),
                                meta->dec_indices.data_ptr<int32_t>(),
@@ -1227,6 +1260,11 @@ torch::Tensor AttentionLayer::forward(const torch::Tensor& qkv, const torch::Ten
               "positions and out_loc must be int32 for the fused pass");
   TORCH_CHECK(batch.out_loc.size(0) == qkv.size(0) && positions.size(0) == qkv.size(0),
               "positions and out_loc need one entry per token");
+  if (backend_->decode_layer_fits(qkv, batch))
+    return backend_->decode_layer(qkv, positions, q_norm_ ? q_norm_->weight.data_ptr() : nullptr,
+                                  k_norm_ ? k_norm_->weight.data_ptr() : nullptr,
+                                  q_norm_ ? q_norm_->eps() : 0.f, rotary_->cos_cache(),
+                                  rotary_->sin_cache(), layer_id_, batch);
   auto kc = backend_->kv_cache()->k_cache(layer_id_);
   auto vc = backend_->kv_cache()->v_cache(layer_id_);
   check_sgl(sgl_fused_qknorm_rope_store(

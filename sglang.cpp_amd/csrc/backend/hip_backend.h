@@ -131,6 +131,16 @@ class HipAttnBackend : public BaseAttnBackend {
   // [T, Hq * D].
   torch::Tensor attend(const torch::Tensor& q, int layer_id, Batch& batch);
 
+  // Norm, RoPE, store and attention of a decode batch's tokens in one call
+  // (sgl_decode_layer): qkv [batch, (Hq + 2 Hkv) D], its q part rotated in place;
+  // null weights: no norm. Returns [batch, Hq * D]. decode_layer_fits: the
+  // batch is one it takes (a decode batch whose query row i is token i).
+  bool decode_layer_fits(const torch::Tensor& qkv, Batch& batch) const;
+  torch::Tensor decode_layer(const torch::Tensor& qkv, const torch::Tensor& positions,
+                             const void* q_weight, const void* k_weight, float eps,
+                             const torch::Tensor& cos, const torch::Tensor& sin, int layer_id,
+                             Batch& batch);
+
   // Mixed batches: one launch with the decode rows on a share of the CUs and
   // the prefill rows on the others (default on, for kv-head counts dividing
   // 8); otherwise, with overlap_mixed, the prefill rows on a side stream
@@ -148,6 +158,8 @@ class HipAttnBackend : public BaseAttnBackend {
  private:
   std::shared_ptr<HipAttnMetadata> metadata_of(Batch& batch) const;
   torch::Tensor& workspace(int64_t bytes);
+  // The split workspace of a decode launch with this metadata.
+  torch::Tensor& decode_workspace(const HipAttnMetadata& meta, void* stream);
   torch::Tensor to_device(const std::vector<int32_t>& host, HipAttnMetadata& meta);
 
   void prepare_mixed_for_capture(Batch& batch);

@@ -22,6 +22,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "norm_rope_row.h"
 
 namespace sgl {
 namespace {
@@ -44,17 +45,6 @@ __device__ __forceinline__ void rmsnorm8(float (&x)[8], const uint16_t* __restri
 #pragma unroll
   for (int i = 0; i < 8; ++i) x[i] = round_t<DT>((x[i] * scale) * wf[i]);
 }
-
-// One rotated value: x c + p' s, p' the partner with its sign flipped on
-// the first half (x c - p s there: negation is exact), as one multiply and
-// one fused multiply-add wherever RoPE is applied, so every path rounds
-// alike.
-__device__ __forceinline__ float rope_one(float x, float p_signed, float c, float s) {
-  return fmaf(p_signed, s, x * c);
-}
-
-// Sign bits of both 16-bit halves of a packed word (bf16 and fp16 alike).
-constexpr uint32_t kSign2 = 0x80008000u;
 
 // Rotate-half RoPE of the 8 values this lane holds; x must hold DT values.
 template <int LPR, int DT>
@@ -321,50 +311,15 @@ __global__ void __launch_bounds__(256) fused_qknorm_rope_store_kernel(
   float wf[8];
   if (w != nullptr) unpack8(ldg128(w + lane_in_row * 8), wf);
   const bool first = lane_in_row < HALF;
-  const uint32_t psign = first ? kSign2 : 0u;
   const int jj = first ? lane_in_row : lane_in_row - HALF;
-  f32x4_t c0[NT], c1[NT], s0[NT], s1[NT];
+  RopeRow rope[NT];
+#pragma unroll
+  for (int k = 0; k < NT; ++k)
+    rope[k] = load_rope_row(cos_cache + pos[k] * (D / 2) + jj * 8,
+                            sin_cache + pos[k] * (D / 2) + jj * 8);
 #pragma unroll
   for (int k = 0; k < NT; ++k) {
-    const float* cr = cos_cache + pos[k] * (D / 2) + jj * 8;
-    const float* sr = sin_cache + pos[k] * (D / 2) + jj * 8;
-    c0[k] = *reinterpret_cast<const f32x4_t*>(cr);
-    c1[k] = *reinterpret_cast<const f32x4_t*>(cr + 4);
-    s0[k] = *reinterpret_cast<const f32x4_t*>(sr);
-    s1[k] = *reinterpret_cast<const f32x4_t*>(sr + 4);
-  }
-#pragma unroll
-  for (int k = 0; k < NT; ++k) {
-    float x[8];
-    unpack8(raw[k], x);
-    u32x4_t words = raw[k];
-    if (w != nullptr) {
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
-      ss = group_sum<LPR>(ss);
-      const float scale = rsqrtf(ss * (1.0f / D) + eps);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        words[i] = pack_bf16x2((x[2 * i] * scale) * wf[2 * i], (x[2 * i + 1] * scale) * wf[2 * i + 1]);
-      unpack8(words, x);
-    }
-    float p[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t wd = words[i];
-      uint32_t pw;
-      if constexpr (HALF == 8) pw = dpp_u32<0x128>(wd);
-      else pw = static_cast<uint32_t>(__shfl_xor(static_cast<int>(wd), HALF, kWave));
-      pw ^= psign;
-      p[2 * i] = bf16_lo(pw);
-      p[2 * i + 1] = bf16_hi(pw);
-    }
-    const float c[8] = {c0[k][0], c0[k][1], c0[k][2], c0[k][3], c1[k][0], c1[k][1], c1[k][2], c1[k][3]};
-    const float sn[8] = {s0[k][0], s0[k][1], s0[k][2], s0[k][3], s1[k][0], s1[k][1], s1[k][2], s1[k][3]};
-#pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = rope_one(x[i], p[i], c[i], sn[i]);
-    const u32x4_t packed = pack8(x);
+    const u32x4_t packed = norm_rope_row<LPR>(raw[k], w != nullptr, wf, eps, first, rope[k]);
     if (tb * NT + k < num_tokens) {
       if (is_q || k_back) stg128_nt<kFusedNtStore>(rowb[k] + lane_off, packed);
       if (!is_q) stg128_nt<kFusedNtStore>(k_cache + slot[k] * hkv * D + (static_cast<uint32_t>((r - hq) * D) + head_off), packed);

@@ -943,3 +943,88 @@ def test_prefill_empty_kv_rows_are_zero(oracle, dev):
     ref = oracle.prefill(u16(q[:300]).copy(), u16(kc), u16(vc), b.indices[:300], qo[:2], kvp[:2],
                          1 / math.sqrt(128))
     assert_attn_close(got[:300], ref, what="neighbour of the empty request")
+
+
+def _decode_layer_case(dev, hq, hkv, lens, norm, seed, unknown=False, alias=None, stray=None):
+    """Inputs of a decode step; alias = (request, position, other request): the
+    first one's slot there becomes the other's new slot; stray: a request whose
+    out_loc is not among its own slots."""
+    rng = np.random.default_rng(seed)
+    b = wl.make_paged_batch(rng, [max(0, n - 1) for n in lens], lens, page_size=16, decode=True,
+                            spare_pages=2)
+    loc = np.array([b.page_table[r, max(0, n - 1)] for r, n in enumerate(lens)], np.int32)
+    idx = b.indices.copy()
+    if alias is not None:
+        r, at, other = alias
+        idx[b.kv_indptr[r] + at] = loc[other]
+    if stray is not None:
+        loc[stray] = b.num_slots - 1
+    g = gen(dev, seed)
+    kc, vc = (randn_bf16((b.num_slots, hkv, 128), dev, g) for _ in range(2))
+    B = len(lens)
+    qkv = randn_bf16((B, (hq + 2 * hkv) * 128 + 64), dev, g)[:, :(hq + 2 * hkv) * 128]
+    w = [(torch.rand(128, device=dev, generator=g) + 0.5).to(torch.bfloat16) if norm else None
+         for _ in range(2)]
+    cos, sin = capi.rope_cos_sin_cache(20_000, 128, 1e6, dev)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(dev)
+    plan = capi.decode_plan(b.kv_indptr, hq, hkv, 128)
+    if unknown:
+        plan.max_request_tokens = 0
+    pos = t([max(0, n - 1) for n in lens])
+    return plan, qkv, kc, vc, w, cos, sin, pos, t(loc), t(idx), t(b.kv_indptr)
+
+
+@pytest.mark.parametrize("hq,hkv,lens,norm,unknown,alias,stray", [
+    (16, 8, [512, 400, 1, 17], True, False, None, None),
+    (16, 8, [512, 400, 1, 17], False, False, None, None),
+    (32, 8, [800], True, False, None, None),
+    (32, 8, [801, 3], True, False, None, None),            # two launches
+    (64, 4, [16, 15, 33], True, False, None, None),        # G = 16
+    (8, 8, [64, 0, 65], True, False, None, None),          # an empty request
+    (8, 1, [9000, 5], True, True, None, None),             # slots past the LDS stage
+    (16, 8, [300, 200, 100], True, False, (0, 150, 2), None),  # reads another's new token
+    (8, 1, [9000, 5], True, True, (0, 8500, 1), None),
+    (16, 8, [300, 200], True, False, (1, 0, 0), 1),
+    (4, 4, [20 + i % 7 for i in range(64)], True, False, (63, 2, 0), None),
+    (4, 4, [20 + i % 7 for i in range(65)], True, False, (64, 2, 0), None),  # two launches
+])
+def test_decode_layer_equals_store_then_decode(dev, hq, hkv, lens, norm, unknown, alias, stray):
+    """One launch for norm, RoPE, store and decode leaves the bits of the store
+    pass followed by the decode: output, rotated q, pool; a request may read a
+    slot that another request of the batch stores in the same step."""
+    note(f"decode layer hq={hq} hkv={hkv} B={len(lens)} norm={norm} alias={alias} stray={stray}")
+    plan, qkv, kc, vc, (qw, kw), cos, sin, pos, loc, idx, kvp = _decode_layer_case(
+        dev, hq, hkv, lens, norm, 41, unknown, alias, stray)
+    ws = capi.decode_workspace(plan, dev)
+    scale = 1 / math.sqrt(128)
+    q2, k2, v2 = qkv.clone(), kc.clone(), vc.clone()
+    o, o2 = (torch.full((len(lens), hq, 128), float("nan"), device=dev, dtype=torch.bfloat16)
+             for _ in range(2))
+    capi.fused_qknorm_rope_store(q2, k2, v2, qw, kw, cos, sin, pos, loc, hq, hkv, 128, 1e-6,
+                                 write_k_back=False)
+    capi.paged_decode(plan, q2[:, :hq * 128].view(len(lens), hq, 128), k2, v2, idx, kvp, o2, ws,
+                      scale)
+    capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, loc, 1e-6, idx, kvp, hq, o, ws,
+                      scale)
+    torch.cuda.synchronize()
+    for got, ref, what in ((qkv, q2, "qkv"), (kc, k2, "k pool"), (vc, v2, "v pool"), (o, o2, "out")):
+        assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), what
+
+
+def test_decode_layer_past_the_plan(dev):
+    """Requests past the plan's capacity: NaN rows and the status, the tokens
+    stored all the same."""
+    note("decode layer past its plan")
+    plan, qkv, kc, vc, (qw, kw), cos, sin, pos, loc, idx, kvp = _decode_layer_case(
+        dev, 16, 8, [100, 40, 500, 30], True, 43)
+    plan = capi.decode_plan(np.array([0, 100, 200, 300, 400], np.int32), 16, 8, 128)
+    k2 = kc.clone()
+    ws = capi.decode_workspace(plan, dev)
+    o = torch.zeros((4, 16, 128), device=dev, dtype=torch.bfloat16)
+    q2 = qkv.clone()
+    capi.fused_qknorm_rope_store(q2, k2, vc.clone(), qw, kw, cos, sin, pos, loc, 16, 8, 128, 1e-6,
+                                 write_k_back=False)
+    capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, loc, 1e-6, idx, kvp, 16, o, ws)
+    assert capi.decode_status(ws) == -3
+    assert not torch.isnan(o[:2].float()).any() and torch.isnan(o[2:].float()).all()
+    assert torch.equal(qkv, q2) and torch.equal(kc, k2)
