@@ -215,12 +215,15 @@ struct HeadState {
 //
 // K and V of step t + 1 are in flight during step t; the Q rows are loaded
 // first and the first step's K/V rows issued before Q is waited for.
-// kQReady: L.q holds the Q rows already.
-template <bool kState, bool kBarrier = !kState, bool kRows = false, bool kQReady = false>
+// kQReady: the Q rows come to L.q in mid(), called with the first step's K/V rows
+// in flight; it returns whether those rows have to be loaded again.
+template <bool kState, bool kBarrier = !kState, bool kRows = false, bool kQReady = false,
+          class Mid = bool (*)()>
 __device__ __forceinline__ void decode_head(const DecodeArgs& a, WaveLds& L, const int32_t* sidx,
                                             int pslot, bool whole, int h, int len, int qrow,
                                             int lane, HeadState* st = nullptr,
-                                            u32x4_t* kt = nullptr, char* oslot = nullptr) {
+                                            u32x4_t* kt = nullptr, char* oslot = nullptr,
+                                            const Mid& mid = Mid{}) {
   const int n = lane & 15;
   const int j = lane >> 4;
   const int G = a.group;
@@ -269,6 +272,13 @@ __device__ __forceinline__ void decode_head(const DecodeArgs& a, WaveLds& L, con
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       *reinterpret_cast<u32x4_t*>(L.q + (u * 4 + j) * kQPitch + n * 8) = qv[u];
+  } else {
+    static_assert(kRows, "the first step's K is loaded as whole rows");
+    if (mid()) {
+      load_v_step(krow, ss_bytes, sidx, 0, len, j, kr);
+      load_v_step(vlane, ss_bytes, sidx, 0, len, j, vr);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
   wave_lds_sync();
 
@@ -713,20 +723,24 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
   const bool staged = len <= kSmallStage;
   if (!skip && staged)
     for (int e = threadIdx.x; e < len; e += blockDim.x) slots[e] = sp[e];
+  RopeRow rope;
   if constexpr (kLayer) {
-    // Row `row`'s k (kv head h) normalised and rotated, or its v, to the pool.
+    const int64_t at = static_cast<int64_t>(new_pos) * (kD / 2) + (l16 & 7) * 8;
+    rope = load_rope_row(nt.cos + at, nt.sin + at);
+  }
+  __syncthreads();  // slots (and the other requests' new slots) staged
+  if (staged) sp = slots;
+  // The new token: normalised, rotated and stored; returns whether other
+  // requests' tokens had to be stored too. Runs with the first K/V rows in
+  // flight, so its barrier waits for them and for the stores at once.
+  auto new_token = [&]() -> bool {
     auto store_kv = [&](const u32x4_t& v, bool is_v, int loc) {
       stg128((is_v ? nt.vc : nt.kc) + (static_cast<int64_t>(loc) * a.hkv + h) * kD + l16 * 8, v);
     };
     float wf[8];
     unpack8(wraw, wf);
-    auto rotated = [&](const u32x4_t& v, int pos) {
-      const int64_t at = static_cast<int64_t>(pos) * (kD / 2) + (l16 & 7) * 8;
-      return norm_rope_row<16>(v, nt.qw != nullptr, wf, nt.eps, l16 < 8,
-                               load_rope_row(nt.cos + at, nt.sin + at));
-    };
     if (vec < G + 1) {
-      const u32x4_t v = rotated(raw, new_pos);
+      const u32x4_t v = norm_rope_row<16>(raw, nt.qw != nullptr, wf, nt.eps, l16 < 8, rope);
       if (vec < G) {
         stg128(nt.qkv + r * nt.qkv_st + (h * G + vec) * kD + l16 * 8, v);
         *reinterpret_cast<u32x4_t*>(ql[0].q + vec * kQPitch + l16 * 8) = v;
@@ -739,34 +753,38 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     for (int e = threadIdx.x; e < (16 - G) * 16; e += blockDim.x)
       *reinterpret_cast<u32x4_t*>(ql[0].q + (G + (e >> 4)) * kQPitch + (e & 15) * 8) =
           u32x4_t{0, 0, 0, 0};
-    __syncthreads();  // slots, Q and the other rows' slots staged; own stores done
     if (a.batch > 1 && !skip) {
       uint64_t seen = 0;
       for (int e = threadIdx.x; e < len; e += blockDim.x) {
-        const int slot = staged ? slots[e] : sp[e];
+        const int slot = sp[e];
         for (int o = 0; o < a.batch; ++o)
           if (locs[o] == slot) seen |= 1ull << o;
       }
       seen &= ~(1ull << r);
-      if (seen != 0)
-        atomicOr(reinterpret_cast<unsigned long long*>(&shared_rows), seen);
-      __syncthreads();
-      uint64_t others = shared_rows;
-      if (others != 0) {
-        for (; others != 0; others &= others - 1) {
-          const int o = __builtin_ctzll(others);
-          if (vec == G || vec == G + 1) {
-            const u32x4_t v = ldg128(nt.qkv + o * nt.qkv_st +
-                                     (a.hq + (vec == G ? 0 : a.hkv) + h) * kD + l16 * 8);
-            if (vec == G) store_kv(rotated(v, nt.positions[o]), false, locs[o]);
-            else store_kv(v, true, locs[o]);
-          }
-        }
-        __syncthreads();
+      if (seen != 0) atomicOr(reinterpret_cast<unsigned long long*>(&shared_rows), seen);
+    }
+    __syncthreads();  // Q in LDS, the stores done
+    const uint64_t others = shared_rows;
+    if (others == 0) return false;
+    for (uint64_t left = others; left != 0; left &= left - 1) {
+      const int o = __builtin_ctzll(left);
+      if (vec == G || vec == G + 1) {
+        const u32x4_t v = ldg128(nt.qkv + o * nt.qkv_st +
+                                 (a.hq + (vec == G ? 0 : a.hkv) + h) * kD + l16 * 8);
+        const int64_t at = static_cast<int64_t>(nt.positions[o]) * (kD / 2) + (l16 & 7) * 8;
+        if (vec == G)
+          store_kv(norm_rope_row<16>(v, nt.qw != nullptr, wf, nt.eps, l16 < 8,
+                                     load_rope_row(nt.cos + at, nt.sin + at)),
+                   false, locs[o]);
+        else
+          store_kv(v, true, locs[o]);
       }
     }
-  }
+    __syncthreads();
+    return true;
+  };
   if (skip) {
+    if constexpr (kLayer) new_token();
     // Past the capacity: NaN rows; empty request: zero rows (G heads of h).
     const uint32_t fill = len <= 0 ? 0u : 0x7fc07fc0u;
     for (int e = threadIdx.x; e < G * (kD / 8); e += blockDim.x) {
@@ -777,10 +795,6 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     }
     return;
   }
-  if (staged) {
-    if constexpr (!kLayer) __syncthreads();
-    sp = slots;
-  }
   const int per = ((len + kSmallWaves - 1) / kSmallWaves + kStep - 1) / kStep * kStep;
   const int t0 = min(len, wave * per);
   const int t1 = min(len, t0 + per);
@@ -789,9 +803,19 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
   st.l = 0.f;
 #pragma unroll
   for (int nb = 0; nb < 8; ++nb) st.acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  if (t0 < t1)
-    decode_head<true, false, true, kLayer>(a, ql[kLayer ? 0 : wave], sp + t0, 0, false, h, t1 - t0,
-                                           qrow, lane, &st, xs.kt[wave]);
+  if constexpr (kLayer) {
+    // The piece's first step holds the new token: its rows were loaded too early.
+    const bool early = t1 == len && t1 - t0 <= kStep;
+    if (t0 < t1)
+      decode_head<true, false, true, true>(a, ql[0], sp + t0, 0, false, h, t1 - t0, qrow, lane, &st,
+                                           xs.kt[wave], nullptr,
+                                           [&]() { return new_token() || early; });
+    else
+      new_token();
+  } else if (t0 < t1) {
+    decode_head<true, false, true>(a, ql[wave], sp + t0, 0, false, h, t1 - t0, qrow, lane, &st,
+                                   xs.kt[wave]);
+  }
   __syncthreads();  // every K tile read before the exchange overwrites them
 #pragma unroll
   for (int nb = 0; nb < 8; ++nb)
