@@ -236,8 +236,10 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
 // count wave-wide from the comparison masks); kCompact: also the copies
 // above cthr, placed element-major (element j of every lane, lanes in
 // order, then element j + 1), a fixed order that needs one lane count per
-// element that has any copy.
-template <bool kCompact>
+// element that has any copy. kFirst: thr is 0 and nothing counts the block (the
+// same mass: max(x, 0) is x above 0 and 0 otherwise, NaN included; the sweep is
+// bound by its vector operations: 256 rows of 151,936 logits 74.7 -> 72.5 us).
+template <bool kCompact, bool kFirst>
 __device__ __forceinline__ void sweep_block(const BlockVals& bv, int b, float thr, float cthr,
                                             float& wm, int& wn, Shared& sh) {
   const int lane = threadIdx.x & 63;
@@ -247,12 +249,16 @@ __device__ __forceinline__ void sweep_block(const BlockVals& bv, int b, float th
 #pragma unroll
     for (int j = 0; j < kVec; ++j) {
       const float x = bv.v[s][j];
-      const bool above = x > thr;
-      m += above ? x : 0.f;
-      wn += __builtin_popcountll(__ballot(above));
+      if constexpr (kFirst) {
+        m += fmaxf(x, 0.f);
+      } else {
+        const bool above = x > thr;
+        m += above ? x : 0.f;
+        wn += __builtin_popcountll(__ballot(above));
+      }
     }
   m = wave_sum_f(m);
-  wm += m;
+  if constexpr (!kFirst) wm += m;
   if (lane == 0) sh.pool[b] = m;
   if constexpr (kCompact) {
     uint64_t mk[kPerLane];
@@ -289,8 +295,9 @@ __device__ __forceinline__ void sweep_block(const BlockVals& bv, int b, float th
 // Block masses, row mass and row count of the probabilities above thr.
 // kCompact: also copy the probabilities above cthr (the caller has zeroed
 // sh.ncand; an overflow shows as sh.ncand > kCandCap). Waves take blocks
-// round-robin, two blocks (8 loads per lane) in flight.
-template <bool kCompact, class Src>
+// round-robin, two blocks (8 loads per lane) in flight. kFirst: the block
+// masses and copies only, for thr = 0.
+template <bool kCompact, bool kFirst, class Src>
 __device__ __forceinline__ void sweep(const Src& row, int d, bool vec, float thr, float cthr,
                                       Shared& sh) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -304,15 +311,16 @@ __device__ __forceinline__ void sweep(const Src& row, int d, bool vec, float thr
     BlockVals x0, x1;
     load_block(row, b, d, true, x0);
     load_block(row, b + kWaves, d, true, x1);
-    sweep_block<kCompact>(x0, b, thr, cthr, wm, wn, sh);
-    sweep_block<kCompact>(x1, b + kWaves, thr, cthr, wm, wn, sh);
+    sweep_block<kCompact, kFirst>(x0, b, thr, cthr, wm, wn, sh);
+    sweep_block<kCompact, kFirst>(x1, b + kWaves, thr, cthr, wm, wn, sh);
   }
   for (; b < nblk; b += kWaves) {
     BlockVals x0;
     load_block(row, b, d, b < nfull, x0);
-    sweep_block<kCompact>(x0, b, thr, cthr, wm, wn, sh);
+    sweep_block<kCompact, kFirst>(x0, b, thr, cthr, wm, wn, sh);
   }
-  finish_totals(wm, wn, sh);
+  if constexpr (kFirst) __syncthreads();
+  else finish_totals(wm, wn, sh);
 }
 
 // The same sweep over the copies: each group of 16 lanes takes one block
@@ -469,9 +477,9 @@ struct StreamSweep {
   const Src& row;
   int d;
   bool vec;
-  template <bool kCompact>
+  template <bool kCompact, bool kFirst = false>
   __device__ __forceinline__ void run(float thr, float cthr, Shared& sh) const {
-    sweep<kCompact>(row, d, vec, thr, cthr, sh);
+    sweep<kCompact, kFirst>(row, d, vec, thr, cthr, sh);
   }
   __device__ __forceinline__ void pick(float thr, float u, Shared& sh) const {
     draw(row, d, vec, thr, u, sh);
@@ -495,7 +503,7 @@ struct HeldSweep {
   __device__ __forceinline__ void pick(float thr, float u, Shared& sh) const {
     draw(row, d, true, thr, u, sh);
   }
-  template <bool kCompact>
+  template <bool kCompact, bool kFirst = false>
   __device__ __forceinline__ void run(float thr, float cthr, Shared& sh) const {
     // Wave-uniform, in a scalar register (block indices and LDS addresses
     // then cost no VGPRs).
@@ -527,12 +535,13 @@ struct HeldSweep {
 #pragma unroll
             for (int j = 0; j < kVec; ++j) bv.v[s][j] = in ? bv.v[s][j] : 0.f;
         }
-        sweep_block<kCompact>(bv, b, thr, cthr, wm, wn, sh);
+        sweep_block<kCompact, kFirst>(bv, b, thr, cthr, wm, wn, sh);
       }
       // One block's values live at a time (the row itself takes 4 NC VGPRs).
       __builtin_amdgcn_sched_barrier(0);
     }
-    finish_totals(wm, wn, sh);
+    if constexpr (kFirst) __syncthreads();
+    else finish_totals(wm, wn, sh);
   }
 };
 
@@ -542,7 +551,8 @@ struct HeldSweep {
 constexpr float kCandThr = 1.f / static_cast<float>(kCandCap - kCandCap / 8);
 
 // The row's draws. kPre: the block masses of the first sweep and, where they
-// fit (pre_cand), its copies are in sh already, its mass and count are not.
+// fit (pre_cand), its copies are in sh already. The first sweep leaves no mass
+// or count of the row: only a first draw that found nothing needs them.
 template <bool kPre, class Src, class Sweep>
 __device__ __forceinline__ void sample_row(const SampleArgs& a, const Src& row, const Sweep& rs,
                                            Shared& sh, bool pre_cand = false) {
@@ -554,10 +564,10 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const Src& row, 
   if (kPre) {
   } else if (cand_ok) {
     if (threadIdx.x == 0) sh.ncand = 0;
-    rs.template run<true>(0.f, cand_thr, sh);
+    rs.template run<true, true>(0.f, cand_thr, sh);
     cand = sh.ncand <= kCandCap;
   } else {
-    rs.template run<false>(0.f, 0.f, sh);
+    rs.template run<false, true>(0.f, 0.f, sh);
   }
   if (a.mode == 0) {
     rs.pick(0.f, u, sh);
@@ -593,8 +603,8 @@ __device__ __forceinline__ void sample_row(const SampleArgs& a, const Src& row, 
       } else {
         rs.template run<false>(pivot, 0.f, sh);
       }
-    } else if (kPre && pivot == 0.f) {
-      rs.template run<false>(0.f, 0.f, sh);  // nothing drawn: the first sweep's mass and count
+    } else if (pivot == 0.f) {
+      rs.template run<false>(0.f, 0.f, sh);  // nothing drawn: the row's mass and count
     }
     q = sh.total;
     const int count = sh.count;
