@@ -515,7 +515,9 @@ int sgl_gelu_and_mul(void* out, const void* input, int64_t tokens, int64_t d,
  * is NULL, the scalar temperature (> 0). logits_dtype: SGL_DTYPE_BF16,
  * SGL_DTYPE_F16 or SGL_DTYPE_F32; row strides in elements (>= vocab). One
  * workgroup per row; aligned 16-bit rows of up to 163,840 elements are
- * held in registers and read from HBM once. Exponentials as
+ * held in registers and read from HBM once. Small batches of long aligned rows
+ * take two launches of many workgroups, with the same bits, unless probs and
+ * logits overlap. Exponentials as
  * 2^(fma(x, a, -max a)) with a = log2e / t (relative error of a probability
  * below ~1e-5 against the exact softmax of float(x) / t). A row whose
  * temperature is not positive gets NaN probabilities.

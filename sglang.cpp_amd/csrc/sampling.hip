@@ -881,7 +881,8 @@ __global__ void __launch_bounds__(kThreads) sampling_split_rounds(SampleArgs a, 
 // against 30.7. What is left is the slowest row's rounds and repeated sweeps,
 // one workgroup's at about 3 and 8 to 10 us each.
 int64_t split_workspace(int64_t batch, int64_t d) {
-  if (batch <= 0 || d < 65536 || d > static_cast<int64_t>(kCandBlocks) * kBlock || batch * 2000 > d)
+  if (batch <= 0 || batch > 80 || d < 65536 ||
+      d > static_cast<int64_t>(kCandBlocks) * kBlock || batch * 2000 > d)
     return 0;
   return batch * split_layout(static_cast<int>(d)).row;
 }

@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(sp::kStatLanes) softmax_write_slices(SoftmaxAr
 // 7.7, x 96 11.9 against 13.1. bf16 rows too long to hold: 200,000 x 64 42.4 ->
 // 28.0, x 160 55.1 against 58.3.
 inline bool split_rows(bool held, int64_t batch, int64_t d) {
-  return d >= (held ? 65536 : 32768) && batch * (held ? 2000 : 1500) <= d;
+  return batch <= 128 && d >= (held ? 65536 : 32768) && batch * (held ? 2000 : 1500) <= d;
 }
 
 // The first launch writes into the probabilities' rows: the logits must lie
@@ -268,7 +268,7 @@ int launch_softmax(const SoftmaxArgs& a, hipStream_t s) {
   const dim3 grid(static_cast<uint32_t>(a.batch));
   const dim3 held(sp::kStatLanes);
   const bool reg_rows = DT != SGL_DTYPE_F32 && per_lane <= kMaxRegChunks;
-  if (a.vec && a.batch <= 0xffff && split_rows(reg_rows, a.batch, a.d) &&
+  if (a.vec && split_rows(reg_rows, a.batch, a.d) &&
       !overlapping<DT>(a)) {
     const int slices = row_slices(a.batch, a.d);
     hipLaunchKernelGGL((softmax_lane_stats<DT>),
