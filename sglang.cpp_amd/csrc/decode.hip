@@ -671,7 +671,9 @@ constexpr int kMaxLayerBatch = 64;  // requests of a sgl_decode_layer launch
 // (h, r) takes request r's q heads of kv head h, its k head and its v head
 // through the norm and RoPE (the store pass's arithmetic, so the same bits),
 // writes q back, stores k and v at out_loc[r] and attends. Its own stores are
-// visible to its waves after the barrier; a row another request of the batch
+// visible to its waves after the barrier, and the first steps, loaded before
+// it, are loaded again where out_loc[r] may be among their slots (the last slot
+// as a rule; the workgroup looks for it elsewhere); a row another request of the batch
 // stores is read here only if that slot is also among this request's slots,
 // which the workgroup looks for, and then stores that row itself first (the
 // same bytes), so that every read sees this step's stores as after a pass of
@@ -688,7 +690,7 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     float xch[34][kSmallWaves][kWave];
   } xs;
   __shared__ int32_t locs[kMaxLayerBatch];
-  __shared__ uint64_t shared_rows;  // requests whose new slot is among this one's slots
+  __shared__ uint64_t shared_rows;  // requests whose new slot is among this one's slots (see new_token)
   auto& xch = xs.xch;
   const int h = blockIdx.x;
   const int r = blockIdx.y;
@@ -734,8 +736,9 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
   __syncthreads();  // slots (and the other requests' new slots) staged
   if (staged) sp = slots;
   // The new token: normalised, rotated and stored; returns whether other
-  // requests' tokens had to be stored too. Runs with the first K/V rows in
-  // flight, so its barrier waits for them and for the stores at once.
+  // requests' tokens had to be stored too, or its own slot is listed before
+  // the request's last place. Runs with the first K/V rows in flight, so its
+  // barrier waits for them and for the stores at once.
   auto new_token = [&]() -> bool {
     auto store_kv = [&](const u32x4_t& v, bool is_v, int loc) {
       stg128((is_v ? nt.vc : nt.kc) + (static_cast<int64_t>(loc) * a.hkv + h) * kD + l16 * 8, v);
@@ -756,20 +759,22 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     for (int e = threadIdx.x; e < (16 - G) * 16; e += blockDim.x)
       *reinterpret_cast<u32x4_t*>(ql[0].q + (G + (e >> 4)) * kQPitch + (e & 15) * 8) =
           u32x4_t{0, 0, 0, 0};
-    if (a.batch > 1 && !skip) {
+    if (!skip) {
       uint64_t seen = 0;
       for (int e = threadIdx.x; e < len; e += blockDim.x) {
         const int slot = sp[e];
+        uint64_t at = 0;
         for (int o = 0; o < a.batch; ++o)
-          if (locs[o] == slot) seen |= 1ull << o;
+          if (locs[o] == slot) at |= 1ull << o;
+        if (e == len - 1) at &= ~(1ull << r);  // its own slot in its usual place
+        seen |= at;
       }
-      seen &= ~(1ull << r);
       if (seen != 0) atomicOr(reinterpret_cast<unsigned long long*>(&shared_rows), seen);
     }
     __syncthreads();  // Q in LDS, the stores done
-    const uint64_t others = shared_rows;
-    if (others == 0) return false;
-    for (uint64_t left = others; left != 0; left &= left - 1) {
+    const uint64_t found = shared_rows;
+    if (found == 0) return false;
+    for (uint64_t left = found & ~(1ull << r); left != 0; left &= left - 1) {
       const int o = __builtin_ctzll(left);
       if (vec == G || vec == G + 1) {
         const u32x4_t v = ldg128(nt.qkv + o * nt.qkv_st +
@@ -807,7 +812,8 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
 #pragma unroll
   for (int nb = 0; nb < 8; ++nb) st.acc[nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   if constexpr (kLayer) {
-    // The piece's first step holds the new token: its rows were loaded too early.
+    // The piece's first step ends the request, usually with the new token: its
+    // rows were loaded too early (new_token finds the slot anywhere else).
     const bool early = t1 == len && t1 - t0 <= kStep;
     if (t0 < t1)
       decode_head<true, false, true, true>(a, ql[0], sp + t0, 0, false, h, t1 - t0, qrow, lane, &st,

@@ -947,8 +947,8 @@ def test_prefill_empty_kv_rows_are_zero(oracle, dev):
 
 def _decode_layer_case(dev, hq, hkv, lens, norm, seed, unknown=False, alias=None, stray=None):
     """Inputs of a decode step; alias = (request, position, other request): the
-    first one's slot there becomes the other's new slot; stray: a request whose
-    out_loc is not among its own slots."""
+    first one's slot there becomes the other's new slot (the other may be the
+    request itself); stray: a request whose out_loc is not among its own slots."""
     rng = np.random.default_rng(seed)
     b = wl.make_paged_batch(rng, [max(0, n - 1) for n in lens], lens, page_size=16, decode=True,
                             spare_pages=2)
@@ -987,6 +987,16 @@ def _decode_layer_case(dev, hq, hkv, lens, norm, seed, unknown=False, alias=None
     (16, 8, [300, 200], True, False, (1, 0, 0), 1),
     (4, 4, [20 + i % 7 for i in range(64)], True, False, (63, 2, 0), None),
     (4, 4, [20 + i % 7 for i in range(65)], True, False, (64, 2, 0), None),  # two launches
+    # a request's own new slot listed before its end too: the first step of its
+    # first piece, of a later piece (300 tokens: 48 a wave, 800: 112, 9000: 1136)
+    # and past a first step
+    (16, 8, [300, 200], True, False, (0, 0, 0), None),
+    (16, 8, [300, 200], True, False, (0, 50, 0), None),
+    (32, 8, [800], True, False, (0, 3, 0), None),
+    (32, 8, [800], True, False, (0, 112 + 15, 0), None),
+    (32, 8, [800], True, False, (0, 112 + 16, 0), None),
+    (8, 1, [9000], True, True, (0, 1136 * 3 + 2, 0), None),
+    (8, 8, [17], True, False, (0, 0, 0), None),
 ])
 def test_decode_layer_equals_store_then_decode(dev, hq, hkv, lens, norm, unknown, alias, stray):
     """One launch for norm, RoPE, store and decode leaves the bits of the store
