@@ -1260,7 +1260,8 @@ torch::Tensor AttentionLayer::forward(const torch::Tensor& qkv, const torch::Ten
               "positions and out_loc must be int32 for the fused pass");
   TORCH_CHECK(batch.out_loc.size(0) == qkv.size(0) && positions.size(0) == qkv.size(0),
               "positions and out_loc need one entry per token");
-  if (backend_->decode_layer_fits(qkv, batch))
+  if (num_qo_heads_ == backend_->num_qo_heads() && num_kv_heads_ == backend_->num_kv_heads() &&
+      head_dim_ == backend_->head_dim() && backend_->decode_layer_fits(qkv, batch))
     return backend_->decode_layer(qkv, positions, q_norm_ ? q_norm_->weight.data_ptr() : nullptr,
                                   k_norm_ ? k_norm_->weight.data_ptr() : nullptr,
                                   q_norm_ ? q_norm_->eps() : 0.f, rotary_->cos_cache(),

@@ -133,8 +133,9 @@ class HipAttnBackend : public BaseAttnBackend {
 
   // Norm, RoPE, store and attention of a decode batch's tokens in one call
   // (sgl_decode_layer): qkv [batch, (Hq + 2 Hkv) D], its q part rotated in place;
-  // null weights: no norm. Returns [batch, Hq * D]. decode_layer_fits: the
-  // batch is one it takes (a decode batch whose query row i is token i).
+  // null weights: no norm; the heads are the backend's. Returns [batch, Hq * D].
+  // decode_layer_fits: the batch is one it takes (a decode batch whose query
+  // row i is token i).
   bool decode_layer_fits(const torch::Tensor& qkv, Batch& batch) const;
   torch::Tensor decode_layer(const torch::Tensor& qkv, const torch::Tensor& positions,
                              const void* q_weight, const void* k_weight, float eps,

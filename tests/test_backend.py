@@ -195,6 +195,24 @@ def test_attention_layer_matches_unfused_modules(dev, sb):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("backend_hq", [16, 64])
+def test_attention_layer_of_other_head_counts_is_refused(dev, sb, backend_hq):
+    """A decode batch through a layer whose query heads are not the backend's
+    raises, as attend does for prefill batches."""
+    note(f"layer 32/8 on a backend of {backend_hq}/8")
+    rng = np.random.default_rng(56)
+    b = wl.make_paged_batch(rng, [19, 4], [20, 5], page_size=16, decode=True)
+    s = Setup(sb, dev, b, backend_hq, 8, 57)
+    rot = sb.RotaryEmbedding(D, D, 8192, 1e6, 0)
+    layer = sb.AttentionLayer(0, 32, 8, D, s.backend, rot, None, None)
+    s.backend.prepare_metadata(s.batch)
+    wide = _randn((2, 80 * D), dev, _gen(dev, 58))  # rows longer than either layout
+    with pytest.raises(RuntimeError, match="num_qo_heads"):
+        layer.forward(wide[:, :48 * D], s.batch.positions, s.batch)
+    torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
 def test_norm_and_rope_modules_fp16(dev, sb):
     """The reference's RMSNorm / fused qk-norm / RotaryEmbedding dispatch fp16
     as well as bf16 (normalization.cu:346-372, rotary_embedding.cu:124-168):
