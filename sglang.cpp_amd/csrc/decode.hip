@@ -990,8 +990,12 @@ __global__ void __launch_bounds__(kLongGroups * 32) decode_merge_long_kernel(Dec
     for (int k = 0; k < kFoldPieces; ++k) {
       const int p = min(c + k, c1 - 1);
       const int64_t pidx = static_cast<int64_t>(p == 0 ? s0 : 2 * (u0 + p)) * a.hq + head;
-      lse[k] = c + k < c1 ? a.part_lse[pidx] : -INFINITY;
+      lse[k] = a.part_lse[pidx];
       v[k] = *reinterpret_cast<const f32x4_t*>(a.part_o + pidx * kD + 4 * lane);
+      if (c + k >= c1) {  // the last piece again: weight 0, and nothing infinite to weigh
+        lse[k] = -INFINITY;
+        v[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
     }
     float mc = m;
 #pragma unroll

@@ -495,6 +495,35 @@ def test_decode_few_long_requests(oracle, dev, hq, hkv, lens, unknown_longest):
     assert_attn_close(o.float().cpu().numpy(), ref, what="few long requests")
 
 
+@pytest.mark.parametrize("hq,hkv,n", [(16, 8, 1100), (32, 8, 5003), (8, 8, 2560)])
+def test_decode_long_fold_keeps_infinities(dev, hq, hkv, n):
+    """Infinite values in V come out infinite from the fold of many pieces, as
+    from the one-launch kernel (a plan that does not know the longest request)."""
+    note(f"decode long fold, infinite values hq={hq} hkv={hkv} n={n}")
+    b = wl.make_paged_batch(np.random.default_rng(36), [n - 1], [n], page_size=16, decode=True)
+    kc, vc = _pool(dev, b.num_slots, hkv, 128, 37)
+    rows = torch.from_numpy(b.indices[3:n - 16:64].astype(np.int64)).to(dev)
+    vc[rows, :, 5] = float("inf")
+    vc[rows, :, 77] = float("-inf")
+    q = randn_bf16((1, hq, 128), dev, gen(dev, 38))
+    out = []
+    for longest in (n, 0):
+        plan = capi.decode_plan(b.kv_indptr, hq, hkv, 128)
+        assert plan.num_units >= 16 and plan.max_request_tokens == n
+        plan.max_request_tokens = longest
+        o = torch.zeros_like(q)
+        capi.paged_decode(plan, q, kc, vc, torch.from_numpy(b.indices).to(dev),
+                          torch.from_numpy(b.kv_indptr).to(dev), o,
+                          capi.decode_workspace(plan, dev), 1 / math.sqrt(128))
+        torch.cuda.synchronize()
+        out.append(o.float())
+    assert (out[1][..., 5] == float("inf")).all() and (out[1][..., 77] == float("-inf")).all()
+    assert (out[0][..., 5] == float("inf")).all() and (out[0][..., 77] == float("-inf")).all()
+    rest = [d for d in range(128) if d not in (5, 77)]
+    assert_attn_close(out[0][..., rest].cpu().numpy(), out[1][..., rest].cpu().numpy(),
+                      what="the finite columns")
+
+
 def test_decode_few_long_requests_past_the_plan(dev):
     """A long request past the plan's capacity: NaN rows and the status."""
     note("decode long request past its plan")
