@@ -112,6 +112,7 @@ __global__ void __launch_bounds__(64 * kFoldWaves) prefill_merge_kernel(PrefillA
     mx = mc;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      if (k + i >= k1) break;  // the last share again: not added, it may hold infinities
       const float wgt = x[i][16] == -INFINITY ? 0.f : exp2f(x[i][16] - mc);
       den += x[i][17] * wgt;
 #pragma unroll

@@ -732,6 +732,34 @@ def test_prefill_planned(oracle, dev, hq, hkv, cached, new):
                                    qop, kvp, o, ws[:-1])
 
 
+@pytest.mark.parametrize("hq,hkv,cached,new", [(32, 8, 9001, 90), (16, 8, 4095, 2), (16, 8, 4600, 2),
+                                               (32, 4, 3000, 65)])
+def test_prefill_fold_keeps_infinities(dev, hq, hkv, cached, new):
+    """Infinite values in V (behind rows every query sees) come out infinite
+    from the fold of kv shares, as from the launch without shares."""
+    note(f"planned prefill, infinite values hq={hq} hkv={hkv} {cached} {new}")
+    b = wl.make_paged_batch(np.random.default_rng(8), [cached], [cached + new], page_size=16)
+    plan, items = capi.prefill_plan(b.qo_indptr, b.kv_indptr, hq, hkv, 128)
+    assert plan.num_merges > 0
+    kc, vc = _pool(dev, b.num_slots, hkv, 128, 9)
+    rows = torch.from_numpy(b.indices[3:cached - 64:64].astype(np.int64)).to(dev)
+    vc[rows, :, 5] = float("inf")
+    vc[rows, :, 77] = float("-inf")
+    q = randn_bf16((new, hq, 128), dev, gen(dev, 10))
+    one, two = (torch.zeros_like(q) for _ in range(2))
+    idx, qop, kvp = (torch.from_numpy(x).to(dev) for x in (b.indices, b.qo_indptr, b.kv_indptr))
+    ws = torch.empty(plan.workspace_bytes, dtype=torch.uint8, device=dev)
+    capi.paged_prefill(q, kc, vc, idx, qop, kvp, new, one)
+    capi.paged_prefill_planned(plan, torch.from_numpy(items.copy()).to(dev), q, kc, vc, idx, qop,
+                               kvp, two, ws)
+    torch.cuda.synchronize()
+    for o in (one, two):
+        assert (o[..., 5] == float("inf")).all() and (o[..., 77] == float("-inf")).all()
+    rest = [d for d in range(128) if d not in (5, 77)]
+    assert_attn_close(two[..., rest].float().cpu().numpy(), one[..., rest].float().cpu().numpy(),
+                      what="the finite columns")
+
+
 @pytest.mark.parametrize("hq,hkv,qo_last", [(16, 8, 100), (32, 4, 32)])
 def test_prefill_split_kv_short_shares(oracle, dev, hq, hkv, qo_last):
     """Launches that leave CUs idle (at most one 64-row item per CU) split
