@@ -607,7 +607,8 @@ int sgl_sampling_from_logits(const void* logits, int64_t logits_stride_row, int 
  * Any of the draws above with a workspace: the statistics and the first sweep
  * of a small batch's rows then run over many workgroups instead of one per
  * row, with the same samples and success flags, bit for bit. Exactly one of
- * probs (fp32 [batch_size, d], contiguous) and logits is given; the fields are
+ * probs (fp32 [batch_size, d], contiguous) and logits is given (an empty batch
+ * may have neither: a logits_stride_row of 0 then means probs); the fields are
  * the arguments of sgl_*_sampling_from_probs and sgl_sampling_from_logits
  * (mode as there). workspace: sgl_sampling_workspace_bytes(batch_size, d)
  * bytes, 16-byte aligned, written before it is read; with NULL, or where that

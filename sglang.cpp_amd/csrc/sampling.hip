@@ -1067,7 +1067,8 @@ extern "C" int sgl_sampling_rows(const sgl_sampling_args_t* in, void* workspace,
                                  int64_t workspace_bytes, void* stream) {
   if (!in || (in->probs && in->logits)) return SGL_ERR_INVALID_ARG;
   SampleArgs a;
-  if (in->probs) {
+  // An empty batch may come with neither pointer; logits have a row stride.
+  if (in->probs || (!in->logits && in->logits_stride_row == 0)) {
     if (in->mode < 0 || in->mode > 3) return SGL_ERR_INVALID_ARG;
     a = base_args(in->probs, in->uniform, in->out, in->mode == 0 ? nullptr : in->success,
                   in->batch_size, in->d, in->mode == 0 ? 1 : in->max_rounds, in->mode);

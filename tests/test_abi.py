@@ -284,3 +284,31 @@ def test_prefill_plan_leaves_full_batches_alone():
     assert call(arr(0, 20), arr(0, 9000), 8) == -3 and plan.num_items == 0
     assert call(arr(0, -1), arr(0, 9000), 8) == -1
     assert call(arr(0, 20), arr(0, -5), 8) == -1
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3])
+def test_sampling_rows_takes_an_empty_batch(mode):
+    """No rows (a tensor without elements has a null pointer): accepted from
+    probabilities and from logits as the draws without a workspace accept them;
+    a batch of rows with neither pointer is not."""
+    lib = capi.lib()
+    def call(batch, rounds, stride):
+        args = capi.SamplingArgs(logits_stride_row=stride, mode=mode, temperature=1.0,
+                                 batch_size=batch, d=1000, max_rounds=rounds)
+        return lib.sgl_sampling_rows(ctypes.byref(args), None, 0, None)
+    null = (None,) * 2
+    from_probs = {
+        0: lambda b, n: lib.sgl_sampling_from_probs(*null, None, b, 1000, 1, None),
+        1: lambda b, n: lib.sgl_top_k_sampling_from_probs(*null, None, None, None, b, 5, 1000, n, 1,
+                                                          None),
+        2: lambda b, n: lib.sgl_top_p_sampling_from_probs(*null, None, None, None, b, 0.5, 1000, n, 1,
+                                                          None),
+        3: lambda b, n: lib.sgl_top_k_top_p_sampling_from_probs(*null, None, None, None, None, b, 5,
+                                                                0.5, 1000, n, 1, None),
+    }[mode]
+    for batch, rounds in ((0, 4), (0, 0), (1, 4), (-1, 4)):
+        assert call(batch, rounds, 0) == from_probs(batch, rounds)
+        assert call(batch, rounds, 1000) == lib.sgl_sampling_from_logits(
+            None, 1000, 0, None, 1.0, None, mode, None, None, 0, None, 0.0, None, None, batch, 1000,
+            rounds, None)
+    assert call(0, 4, 0) == call(0, 4, 1000) == 0 and call(1, 4, 0) == -1

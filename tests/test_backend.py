@@ -555,6 +555,21 @@ def test_sampling_functions_match_c_abi(dev, sb):
 
 
 @pytest.mark.gpu
+def test_draws_of_an_empty_batch(dev, sb):
+    """No rows: every draw returns empty samples and flags."""
+    note("draws of no rows")
+    probs, u1 = torch.empty((0, 1000), device=dev), torch.empty(0, device=dev)
+    u = torch.empty((4, 0), device=dev)
+    assert sb.flashinfer_sample_from_probs(probs, u1, True).shape == (0,)
+    for r in (sb.flashinfer_top_k_sample_from_probs(probs, u, None, 5, True),
+              sb.flashinfer_top_p_sample_from_probs(probs, u, None, 0.5, True),
+              sb.flashinfer_top_k_top_p_sample_from_probs(probs, u, None, 5.0, None, 0.5, True),
+              sb.sample_from_logits(probs.to(torch.bfloat16), u1, u, u1, u1)):
+        assert r[0].shape == r[1].shape == (0,)
+    assert sb.sample_from_logits(probs, u1, u1)[0].shape == (0,)
+
+
+@pytest.mark.gpu
 def test_write_page_table_module(oracle, dev, sb):
     """The reference's CacheManager::write_page_table call (host page list and
     (table_idx, first_page, last_page) tuples, prefill.cc:144-187) writes what
