@@ -331,7 +331,8 @@ int sgl_paged_decode_noalloc(const sgl_decode_plan_t* plan, const void* q,
  * r's, then sgl_paged_decode of the rotated q rows over the pool (k_cache and
  * v_cache [slots, Hkv, D] contiguous), with the same results. Batches of at
  * most 64 requests that sgl_paged_decode takes in one kernel run as one launch
- * here too; others as those two calls.
+ * here too; others as those two calls. Arguments that either call refuses are
+ * refused before anything is written.
  * Replaces: AttentionLayer::forward's norm, RoPE, store and decode
  *           (src/layers/attention_layer.cc:27-47, src/attention/flashinfer_backend.cu:530-595).
  */

@@ -1351,6 +1351,11 @@ void launch_merge(const DecodeArgs& a, hipStream_t s) {
                        s, a);
 }
 
+int workspace_check(const sgl_decode_plan_t* plan, const void* workspace, int64_t bytes) {
+  if (workspace == nullptr || bytes < plan->workspace_bytes) return SGL_ERR_CAPACITY;
+  return aligned16(workspace) ? SGL_OK : SGL_ERR_ALIGNMENT;
+}
+
 // Points the kernel arguments at a workspace of the plan's layout.
 void bind_workspace(DecodeArgs& a, const sgl_decode_plan_t* plan, void* workspace) {
   const WorkspaceLayout w = workspace_layout(plan->num_units, plan->num_qo_heads);
@@ -1412,9 +1417,8 @@ extern "C" int sgl_paged_decode(const sgl_decode_plan_t* plan, const void* q,
   int st = decode_args(plan, q, q_stride_token, q_stride_head, k_cache, v_cache, kv_stride_slot,
                        kv_stride_head, indices, kv_indptr, q_indptr, batch_size, num_qo_heads,
                        num_kv_heads, head_dim, sm_scale, o, o_stride_token, o_stride_head, a);
+  if (st == SGL_OK) st = workspace_check(plan, workspace, workspace_bytes);
   if (st != SGL_OK) return st;
-  if (workspace == nullptr || workspace_bytes < plan->workspace_bytes) return SGL_ERR_CAPACITY;
-  if (!aligned16(workspace)) return SGL_ERR_ALIGNMENT;
   bind_workspace(a, plan, workspace);
   return launch_decode(a, plan, static_cast<hipStream_t>(stream));
 }
@@ -1431,21 +1435,23 @@ extern "C" int sgl_decode_layer(const sgl_decode_plan_t* plan, void* qkv, int64_
   if (!plan || batch_size < 0) return SGL_ERR_INVALID_ARG;
   if (batch_size == 0) return SGL_OK;
   const int64_t slot = static_cast<int64_t>(num_kv_heads) * head_dim;
+  // What the decode refuses is refused before the store writes anything.
   DecodeArgs a;
+  int st = decode_args(plan, qkv, qkv_stride_token, head_dim, k_cache, v_cache, slot, head_dim,
+                       indices, kv_indptr, nullptr, batch_size, num_qo_heads, num_kv_heads, head_dim,
+                       sm_scale, o, o_stride_token, o_stride_head, a);
+  if (st == SGL_OK) st = workspace_check(plan, workspace, workspace_bytes);
+  if (st != SGL_OK) return st;
   const bool one_launch =
-      decode_args(plan, qkv, qkv_stride_token, head_dim, k_cache, v_cache, slot, head_dim, indices,
-                  kv_indptr, nullptr, batch_size, num_qo_heads, num_kv_heads, head_dim, sm_scale, o,
-                  o_stride_token, o_stride_head, a) == SGL_OK &&
-      workspace != nullptr && workspace_bytes >= plan->workspace_bytes && aligned16(workspace) &&
       batch_size <= kMaxLayerBatch && small_batch(a, plan) && cos_cache && sin_cache && positions &&
       out_loc && (q_weight == nullptr) == (k_weight == nullptr) &&
       qkv_stride_token >= (num_qo_heads + 2 * static_cast<int64_t>(num_kv_heads)) * head_dim &&
       aligned16(cos_cache) && aligned16(sin_cache) && aligned16(q_weight) && aligned16(k_weight);
   if (!one_launch) {
-    const int st = sgl_fused_qknorm_rope_store(
-        qkv, qkv_stride_token, k_cache, v_cache, q_weight, k_weight, cos_cache, sin_cache,
-        positions, out_loc, batch_size, num_qo_heads, num_kv_heads, head_dim, eps,
-        SGL_FUSED_NO_K_WRITEBACK, stream);
+    st = sgl_fused_qknorm_rope_store(qkv, qkv_stride_token, k_cache, v_cache, q_weight, k_weight,
+                                     cos_cache, sin_cache, positions, out_loc, batch_size,
+                                     num_qo_heads, num_kv_heads, head_dim, eps,
+                                     SGL_FUSED_NO_K_WRITEBACK, stream);
     if (st != SGL_OK) return st;
     return sgl_paged_decode(plan, qkv, qkv_stride_token, head_dim, k_cache, v_cache, slot, head_dim,
                             indices, kv_indptr, nullptr, batch_size, num_qo_heads, num_kv_heads,

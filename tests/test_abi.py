@@ -232,6 +232,28 @@ def test_paged_decode_rejects_inconsistent_plan():
     assert lib.sgl_paged_decode(*args(plan, plan.workspace_bytes, 132)) == -4
 
 
+def test_decode_layer_refuses_before_it_stores():
+    """What the decode refuses comes back before the store is launched (a launch
+    without a device would return the runtime's error instead)."""
+    plan = capi.decode_plan([0, 100, 300], 16, 8, 128)
+    wide = capi.decode_plan([0, 100, 1300], 16, 8, 128)  # the two-launch route
+    lib = capi.lib()
+    args = lambda pl, ws_bytes, ws=16, ostride_h=128, batch=2, indices=16: (  # noqa: E731
+        ctypes.byref(pl), 16, 32 * 128, 16, 16, 16, 16, 16, 16, 16, 16, ctypes.c_float(1e-6), indices,
+        16, batch, 16, 8, 128, ctypes.c_float(0.1), 16, 16 * 128, ostride_h, ws, ws_bytes, None)
+    for pl in (plan, wide):
+        n = pl.workspace_bytes
+        assert lib.sgl_decode_layer(*args(pl, n - 1)) == -3
+        assert lib.sgl_decode_layer(*args(pl, n, ws=None)) == -3
+        assert lib.sgl_decode_layer(*args(pl, n, ws=24)) == -4
+        assert lib.sgl_decode_layer(*args(pl, n, ostride_h=132)) == -4
+        assert lib.sgl_decode_layer(*args(pl, n, batch=3)) == -3
+        assert lib.sgl_decode_layer(*args(pl, n, indices=None)) == -1
+        bad = capi.DecodePlan.from_buffer_copy(pl)
+        bad.max_total_tokens += 16
+        assert lib.sgl_decode_layer(*args(bad, n)) == -1
+
+
 @pytest.mark.parametrize("hq,hkv,lens", [
     (32, 8, [(17, 2017), (90, 12_000), (33, 5000), (64, 64)]),
     (32, 4, [(300, 9000)]),

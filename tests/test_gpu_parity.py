@@ -1078,6 +1078,22 @@ def test_decode_layer_equals_store_then_decode(dev, hq, hkv, lens, norm, unknown
         assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), what
 
 
+@pytest.mark.parametrize("lens", [[300, 200], [900, 3]])  # one launch, two
+def test_decode_layer_error_leaves_its_inputs(dev, lens):
+    """A refused call writes nothing."""
+    note(f"decode layer refused {lens}")
+    plan, qkv, kc, vc, (qw, kw), cos, sin, pos, loc, idx, kvp = _decode_layer_case(
+        dev, 16, 8, lens, True, 44)
+    ws = capi.decode_workspace(plan, dev)
+    o = torch.zeros((2, 16, 128), device=dev, dtype=torch.bfloat16)
+    before = [t.clone() for t in (qkv, kc, vc)]
+    with pytest.raises(capi.SglError):
+        capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, loc, 1e-6, idx, kvp, 16, o,
+                          ws[:-16])
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(before, (qkv, kc, vc))) and not o.any()
+
+
 def test_decode_layer_past_the_plan(dev):
     """Requests past the plan's capacity: NaN rows and the status, the tokens
     stored all the same."""
