@@ -329,7 +329,9 @@ int sgl_paged_decode_noalloc(const sgl_decode_plan_t* plan, const void* q,
  * The attention layer's decode step: sgl_fused_qknorm_rope_store (with
  * SGL_FUSED_NO_K_WRITEBACK) on the batch's tokens, token r of qkv being request
  * r's, then sgl_paged_decode of the rotated q rows over the pool (k_cache and
- * v_cache [slots, Hkv, D] contiguous), with the same results. Batches of at
+ * v_cache [slots, Hkv, D] contiguous), with the same results, except for
+ * requests that share an out_loc (which of their tokens that slot then holds is
+ * open in both). Batches of at
  * most 64 requests that sgl_paged_decode takes in one kernel run as one launch
  * here too; others as those two calls. Arguments that either call refuses are
  * refused before anything is written.

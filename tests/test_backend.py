@@ -160,6 +160,27 @@ def test_backend_rejects_fp16_q(dev, sb):
         s.backend.attend(s.q.to(torch.float16), 0, s.batch)
 
 
+def _decode_layer_modules(sb, dev, backend, hq, hkv, seed, norm, layer_id=1):
+    g = _gen(dev, seed)
+    rot = sb.RotaryEmbedding(D, D, 8192, 1e6, 0)
+    qn = kn = None
+    if norm:
+        qn, kn = sb.RMSNorm(D, 1e-6, 0), sb.RMSNorm(D, 1e-6, 0)
+        qn.weight = _randn((D,), dev, g, 0.5) + 1
+        kn.weight = _randn((D,), dev, g, 0.5) + 1
+    return rot, qn, kn, sb.AttentionLayer(layer_id, hq, hkv, D, backend, rot, qn, kn)
+
+
+def _store_then_attend(cache, backend, rot, qn, kn, qkv, batch, hq, hkv, layer=1):
+    """The fused store pass, then attend (q rotated in place in qkv)."""
+    shape = (-1, hkv, D)
+    capi.fused_qknorm_rope_store(
+        qkv, cache.k_cache(layer).view(shape), cache.v_cache(layer).view(shape),
+        None if qn is None else qn.weight, None if kn is None else kn.weight, rot.cos_cache(),
+        rot.sin_cache(), batch.positions, batch.out_loc, hq, hkv, D, 1e-6, write_k_back=False)
+    return backend.attend(qkv[:, :hq * D].view(-1, hq, D), layer, batch)
+
+
 @pytest.mark.gpu
 def test_attention_layer_matches_unfused_modules(dev, sb):
     """AttentionLayer (fused qk-norm + RoPE + store, then attention) equals the
@@ -192,6 +213,126 @@ def test_attention_layer_matches_unfused_modules(dev, sb):
     torch.cuda.synchronize()
     assert torch.equal(o1.view(torch.int16), o2.view(torch.int16))
     assert torch.equal(s1.cache.buffer().view(torch.int16), s2.cache.buffer().view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("norm", [True, False])
+@pytest.mark.parametrize("hq,hkv,lens", [
+    (16, 8, [512, 400, 1, 17]),        # one launch
+    (32, 8, [801, 30]),                # two: a long request
+    (32, 4, [60 + i for i in range(65)]),  # two: past the one-launch batch
+])
+def test_attention_layer_decode_matches_store_then_attend(dev, sb, hq, hkv, lens, norm):
+    """A decode batch through AttentionLayer leaves the bits of the store pass
+    followed by attend: output, rotated q, pool."""
+    note(f"attention layer decode {hq}/{hkv} B={len(lens)} norm={norm}")
+    b = wl.make_paged_batch(np.random.default_rng(60), [n - 1 for n in lens], lens, page_size=16,
+                            decode=True)
+    s1, s2 = (Setup(sb, dev, b, hq, hkv, 61) for _ in range(2))
+    rot, qn, kn, layer = _decode_layer_modules(sb, dev, s1.backend, hq, hkv, 62, norm)
+    qkv = torch.cat([s1.q, s1.k, s1.v], dim=1)
+    qkv1 = qkv.clone()
+    s1.backend.prepare_metadata(s1.batch)
+    o1 = layer.forward(qkv1, s1.batch.positions, s1.batch)
+    s2.backend.prepare_metadata(s2.batch)
+    o2 = _store_then_attend(s2.cache, s2.backend, rot, qn, kn, qkv, s2.batch, hq, hkv)
+    torch.cuda.synchronize()
+    for got, ref in ((o1, o2), (qkv1[:, :hq * D], qkv[:, :hq * D]),
+                     (s1.cache.buffer(), s2.cache.buffer())):
+        assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("max_seq", [1024, 4096])  # one launch a layer at 8 rows, two
+def test_attention_layer_decode_captured_and_padded(dev, sb, max_seq):
+    """AttentionLayer's decode step captured once and replayed on full and
+    padded batches (dummies on a spare row that all store to its slot), eager
+    work in between: each real row is the eager store-then-attend's, and of the
+    pool only the real tokens' slots and the spare slot change."""
+    note(f"attention layer captured decode max_seq={max_seq}")
+    hq, hkv, bs = 16, 8, 8
+    rng = np.random.default_rng(63)
+    full = wl.make_paged_batch(rng, [max_seq - 1] * bs, [max_seq] * bs, page_size=16, decode=True)
+    pt, spare, spare_row = full.page_table, full.num_pages * 16, bs
+    g = _gen(dev, 64)
+    caches = [sb.MHAKVCache(hkv, 1, D, full.num_pages + 1, 16, 0) for _ in range(2)]
+    caches[0].buffer().copy_(_randn(tuple(caches[0].buffer().shape), dev, g))
+    table = torch.from_numpy(pt).to(dev)
+    backends = [sb.HipAttnBackend(c, hq, hkv, D) for c in caches]
+    for be in backends:
+        be.set_page_table(table)
+    be = backends[0]
+    be.init_capture_graph(max_seq, [bs])
+    rot, qn, kn, layer = _decode_layer_modules(sb, dev, be, hq, hkv, 65, True, layer_id=0)
+    qkv = torch.zeros((bs, (hq + 2 * hkv) * D), device=dev, dtype=torch.bfloat16)
+    pos = torch.zeros(bs, dtype=torch.int32, device=dev)
+    loc = torch.from_numpy(np.array([spare + i for i in range(bs)], np.int32)).to(dev)
+    cap = sb.Batch(False, [sb.Req(i, max_seq - 1, max_seq) for i in range(bs)], pos, loc)
+    be.prepare_for_capture(cap)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        layer.forward(qkv, pos, cap)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer.forward(qkv, pos, cap)
+    slots = lambda c: c.buffer().view(2, -1, hkv, D)  # noqa: E731  (K then V, one layer)
+    for lens in ([max_seq] * bs, [5, 700, 33], [1, 16, 17, 400, 800, 64], [max_seq - 3], [9] * bs):
+        n = len(lens)
+        reqs = [sb.Req(i, m - 1, m) for i, m in enumerate(lens)]
+        new = [int(pt[i, m - 1]) for i, m in enumerate(lens)]
+        t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)  # noqa: E731
+        b = sb.Batch(False, reqs + [sb.Req(spare_row, 0, 1)] * (bs - n),
+                     t([m - 1 for m in lens] + [0] * (bs - n)), t(new + [spare] * (bs - n)))
+        caches[1].buffer().copy_(caches[0].buffer())
+        before = slots(caches[0]).clone()
+        be.prepare_metadata(b)
+        be.prepare_for_replay(b)
+        x = _randn((bs, (hq + 2 * hkv) * D), dev, g)
+        qkv.copy_(x), pos.copy_(b.positions), loc.copy_(b.out_loc)
+        graph.replay()
+        torch.cuda.synchronize()
+        eb = sb.Batch(False, reqs, b.positions[:n], b.out_loc[:n])
+        backends[1].prepare_metadata(eb)
+        ref = _store_then_attend(caches[1], backends[1], rot, qn, kn, x[:n], eb, hq, hkv, layer=0)
+        torch.cuda.synchronize()
+        assert torch.equal(qkv[:n, :hq * D].view(torch.int16), x[:n, :hq * D].view(torch.int16))
+        changed = (slots(caches[0]) != before).flatten(2).any(2).any(0).nonzero().flatten().tolist()
+        assert set(changed) <= set(new) | {spare}
+        assert torch.equal(slots(caches[0])[:, new], slots(caches[1])[:, new])
+        assert torch.isfinite(out.float()).all()
+        # Another split of the tokens than the eager plan's: P is rounded to
+        # bf16 against other reference points, so close and not equal.
+        assert_attn_close(out[:n].float().cpu().numpy(), ref.float().cpu().numpy(),
+                          what=f"captured layer {lens}")
+
+
+@pytest.mark.gpu
+def test_attention_layer_planned_prefill_eager_and_captured(oracle, dev, sb):
+    """A few new tokens behind long prefixes take the planned prefill through
+    the backend: against the oracle, and the same metadata recorded in a graph
+    gives the same bits on every replay, with eager batches in between."""
+    note("planned prefill through the backend")
+    hq, hkv = 32, 8
+    b = wl.make_paged_batch(np.random.default_rng(66), [2000, 9001, 500], [2017, 9091, 533],
+                            page_size=16)
+    plan, _ = capi.prefill_plan(b.qo_indptr, b.kv_indptr, hq, hkv, D)
+    assert plan.num_items > 0 and plan.num_merges > 0
+    s = Setup(sb, dev, b, hq, hkv, 67)
+    eager = _run_forward(oracle, s, layer=1)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = s.backend.forward(s.q, s.k, s.v, 1, s.batch)
+    for i in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16)), i
+        again = s.backend.forward(s.q, s.k, s.v, 1, s.batch)  # eager, another workspace
+        torch.cuda.synchronize()
+        assert torch.equal(again.view(torch.int16), eager.view(torch.int16)), i
 
 
 @pytest.mark.gpu

@@ -1078,6 +1078,44 @@ def test_decode_layer_equals_store_then_decode(dev, hq, hkv, lens, norm, unknown
         assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), what
 
 
+def test_decode_layer_padding_rows_cost_like_others(dev):
+    """Rows that share one spare slot (a padded batch's dummies) do not store
+    for each other: 32 of them take about as long as 32 rows with slots of
+    their own, where one row after the other took several times that."""
+    note("decode layer, 32 rows on one slot")
+    hq, hkv, B = 32, 8, 32
+    plan, qkv, kc, vc, (qw, kw), cos, sin, pos, loc, idx, kvp = _decode_layer_case(
+        dev, hq, hkv, [1] * B, True, 45)
+    ws = capi.decode_workspace(plan, dev)
+    o = torch.zeros((B, hq, 128), device=dev, dtype=torch.bfloat16)
+    shared_loc, shared_idx = torch.full_like(loc, int(loc[0])), torch.full_like(idx, int(loc[0]))
+
+    def once(l, i):
+        capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, l, 1e-6, i, kvp, hq, o, ws)
+
+    def us(l, i):
+        once(l, i)
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            for _ in range(50):
+                once(l, i)
+        best = float("inf")
+        for _ in range(10):
+            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            t0.record()
+            graph.replay()
+            t1.record()
+            torch.cuda.synchronize()
+            best = min(best, t0.elapsed_time(t1) * 1000 / 50)
+        return best
+
+    own, shared = us(loc, idx), us(shared_loc, shared_idx)
+    print(f"[case] own slots {own:.2f} us, one slot {shared:.2f} us", flush=True)
+    assert shared < 1.5 * own + 1.0
+
+
 @pytest.mark.parametrize("lens", [[300, 200], [900, 3]])  # one launch, two
 def test_decode_layer_error_leaves_its_inputs(dev, lens):
     """A refused call writes nothing."""
