@@ -1522,23 +1522,19 @@ extern "C" int sgl_paged_mixed(const sgl_decode_plan_t* plan, const void* q,
   if (workspace == nullptr || workspace_bytes < plan->workspace_bytes) return SGL_ERR_CAPACITY;
   if (!aligned16(workspace)) return SGL_ERR_ALIGNMENT;
   bind_workspace(d, plan, workspace);
-  pf::PrefillArgs p;
+  pf::PrefillArgs p{};
   st = pf::prefill_args(q, q_stride_token, q_stride_head, k_cache, v_cache, kv_stride_slot,
                         kv_stride_head, pre_indices, pre_qo_indptr, pre_kv_indptr, pre_q_start,
                         num_qo_heads, num_kv_heads, head_dim, sm_scale, o, o_stride_token,
                         o_stride_head, p);
   if (st != SGL_OK) return st;
   // The prefill role: 8-wave items of 256 packed rows (unpaired, heavy first).
-  const int64_t rows_max = static_cast<int64_t>(pre_max_qo_len) * p.group;
-  const int64_t tiles = pf::launch_tiles((rows_max + 255) / 256, num_kv_heads);
-  const int64_t items = tiles * num_kv_heads * pre_batch;
+  const int64_t items = pf::unpaired_items(p, pre_max_qo_len, 256, pre_batch);
   const int upw = 8 / num_kv_heads;
   // Decode workgroups rounded to a multiple of the 8 XCDs, so the prefill
   // items keep their XCD-aware placement.
   const int64_t dec_blocks = ((plan->num_units + upw - 1) / upw + 7) / 8 * 8;
   if (items + dec_blocks > 0x7fffffff) return SGL_ERR_INVALID_ARG;
-  p.tiles_per_req = static_cast<int>(tiles);
-  p.batch = pre_batch;
   size_t lds = static_cast<size_t>(upw) * unit_lds_bytes<true>(num_kv_heads, plan->kv_chunk_size);
   if (lds < static_cast<size_t>(pf::prefill_lds_bytes<8, 1>()))
     lds = pf::prefill_lds_bytes<8, 1>();

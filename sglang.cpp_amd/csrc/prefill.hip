@@ -178,7 +178,7 @@ extern "C" int sgl_paged_prefill(const void* q, int64_t q_stride_token, int64_t 
   if (batch_size < 0 || max_qo_len < 0 || num_qo_heads <= 0 || num_kv_heads <= 0)
     return SGL_ERR_INVALID_ARG;
   if (batch_size == 0 || max_qo_len == 0) return SGL_OK;
-  PrefillArgs a;
+  PrefillArgs a{};
   const int st = prefill_args(q, q_stride_token, q_stride_head, k_cache, v_cache, kv_stride_slot,
                               kv_stride_head, indices, qo_indptr, kv_indptr, q_start,
                               num_qo_heads, num_kv_heads, head_dim, sm_scale, o,
@@ -204,11 +204,10 @@ extern "C" int sgl_paged_prefill(const void* q, int64_t q_stride_token, int64_t 
   const bool split_kv = !wide && ((rows_max + 63) / 64) * num_kv_heads * batch_size <=
                                      static_cast<int64_t>(device_cus());
   const int bm = wide ? 256 : split_kv ? 64 : 128;
-  const int64_t tiles = pair ? pairs : launch_tiles((rows_max + bm - 1) / bm, num_kv_heads);
-  const int64_t items = tiles * num_kv_heads * batch_size;
+  const int64_t items = pair ? pairs * num_kv_heads * batch_size
+                             : unpaired_items(a, max_qo_len, bm, batch_size);
   if (items > 0x7fffffff) return SGL_ERR_INVALID_ARG;
-  a.tiles_per_req = static_cast<int>(tiles);
-  a.batch = batch_size;
+  if (pair) a.tiles_per_req = static_cast<int>(pairs);
   const dim3 grid(static_cast<uint32_t>(items));
   const hipStream_t s = static_cast<hipStream_t>(stream);
   if (pair)
@@ -354,7 +353,7 @@ extern "C" int sgl_paged_prefill_planned(
   if (!plan || !items || plan->num_items <= 0 || plan->num_merges < 0) return SGL_ERR_INVALID_ARG;
   if (num_qo_heads != plan->num_qo_heads || num_kv_heads != plan->num_kv_heads)
     return SGL_ERR_INVALID_ARG;
-  PrefillArgs a;
+  PrefillArgs a{};
   int st = prefill_args(q, q_stride_token, q_stride_head, k_cache, v_cache, kv_stride_slot,
                         kv_stride_head, indices, qo_indptr, kv_indptr, q_start, num_qo_heads,
                         num_kv_heads, head_dim, sm_scale, o, o_stride_token, o_stride_head, a);

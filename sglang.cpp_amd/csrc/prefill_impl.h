@@ -32,9 +32,9 @@ struct PrefillArgs {
   float scale_log2;
   uint16_t* o;
   int64_t o_st, o_sh;
-  int tiles_per_req;  // query tiles (or pairs) per (request, kv head), see launch_tiles
+  int tiles_per_req;  // query tiles (or pairs) per (request, kv head)
   int num_kv_heads;
-  int batch;
+  int batch, even_tokens;  // unpaired launches, see unpaired_items
   // Planned launches (prefill_item kList): item lin / Hkv = {request, first
   // packed row << 4 | waves of rows, first kv tile, end kv tile | kPartial}, kv
   // head lin % Hkv; partial items leave their state in part[lin].
@@ -326,6 +326,11 @@ __device__ __forceinline__ void pv_steps(const LaneAddr& la, const bf16x8_t (&po
 // tiles in flight then share one or two requests' K/V in L2 (every request's
 // heaviest tiles at a time: 180 us below). Suits launches of several
 // workgroups per CU, which the dispatcher balances.
+// Requests of like lengths (unpaired_items) go rank by rank instead, every
+// request's heaviest tile first: the last request's heavy tiles would start
+// late and run alone at the end, and there is little to gain from L2 (us, one
+// request after the other -> rank by rank: 16q/8kv, 2 x 2048 tokens 66 -> 54, 4 x
+// 1000 38.4 -> 30; 32q/8kv, 2 x 1000 38.9 -> 31; 16q/2kv, 4 x 2048 108 -> 78).
 // Giving each XCD a contiguous share of the (request, head, tile) list left
 // the XCDs of the long requests working alone: 12 prompts of 31 to 1500
 // tokens, 32q/8kv, 224 -> 167 us a layer (its store, 43 us, included).
@@ -360,32 +365,55 @@ constexpr int prefill_lds_bytes() {
   return ring > xch ? ring : xch;
 }
 
-// Query tiles per (request, kv head) an unpaired launch is laid out for: the
-// longest request's, in whole rounds of the XCDs that share a head.
-inline int64_t launch_tiles(int64_t tiles, int num_kv_heads) {
-  const int64_t m = num_kv_heads < kXcds && kXcds % num_kv_heads == 0 ? kXcds / num_kv_heads : 1;
-  return (tiles + m - 1) / m * m;
+// Lays an unpaired launch out for requests of up to max_qo tokens in tiles of
+// tile_rows packed rows and returns its items: per (request, kv head) the longest
+// request's tiles, in whole rounds of the XCDs that share a head.
+// even_tokens: the batch's tokens from which its tiles go rank by rank. They do in
+// batches whose mean length is at least 0.9 of max_qo, up to 1536 items (6 a
+// CU). Below that mean the order by request is the better one more and more
+// often (at 0.75, 32q/8kv, 2 requests up to 4096 tokens: 196 us against 241),
+// and so it is for many items, whose last ones weigh little (64q/4kv, 12 x 700
+// tokens, 2112 items: 167 against 191; 16q/16kv, 16 x 1000 behind 2048, 2048
+// items: 419 against 471).
+inline int64_t unpaired_items(PrefillArgs& a, int max_qo, int tile_rows, int batch) {
+  const int H = a.num_kv_heads;
+  const int64_t m = H < kXcds && kXcds % H == 0 ? kXcds / H : 1;
+  const int64_t tiles = (static_cast<int64_t>(max_qo) * a.group + tile_rows - 1) / tile_rows;
+  const int64_t per_req = (tiles + m - 1) / m * m, items = per_req * H * batch;
+  const int64_t even = (9 * static_cast<int64_t>(max_qo) * batch + 9) / 10;
+  a.tiles_per_req = static_cast<int>(per_req);
+  a.batch = batch;
+  a.even_tokens = batch > 1 && items <= 1536 && even < 0x7fffffff ? static_cast<int>(even) : 0x7fffffff;
+  return items;
 }
 
 // Request, kv head and query tile of item `lin` of an unpaired launch
 // (batch x Hkv x tiles_per_req items).
 __device__ __forceinline__ void item_of(const PrefillArgs& a, int lin, int& r, int& h, int& tile) {
-  const int H = a.num_kv_heads, T = a.tiles_per_req;
+  const int H = a.num_kv_heads;
+  int j, m = 1, x = 0;
   if (H < kXcds && kXcds % H == 0) {
-    const int m = kXcds / H;  // XCDs per head, consecutive ones
-    const int x = lin % kXcds, j = lin / kXcds;
-    r = j / (T / m);
-    const int rank = j - r * (T / m);
+    m = kXcds / H;  // XCDs per head, consecutive ones
+    x = lin % kXcds;
+    j = lin / kXcds;
     h = x / m;
-    tile = T - 1 - (rank * m + x % m);
+    x -= h * m;
   } else {
     // Multiples of 8 heads: head h on XCD h % 8. Other counts: the same
     // order, the heads wherever they fall.
-    const int j = lin / H;
-    r = j / T;
+    j = lin / H;
     h = lin - j * H;
-    tile = T - 1 - (j - r * T);
   }
+  const int ranks = a.tiles_per_req / m;
+  int rank;
+  if (a.qo_indptr[a.batch] - a.qo_indptr[0] >= a.even_tokens) {
+    rank = j / a.batch;
+    r = j - rank * a.batch;
+  } else {
+    r = j / ranks;
+    rank = j - r * ranks;
+  }
+  tile = a.tiles_per_req - 1 - (rank * m + x);
 }
 
 // kList = true (W = 8, KS = 1): the items and their kv shares come from a
@@ -818,7 +846,7 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
 
 // Checks shared by the prefill entry points (pointers, head layout,
 // strides, alignment); fills the kernel arguments except the item layout
-// (tiles_per_req, num_kv_heads).
+// (tiles_per_req, batch, even_tokens or items, part).
 inline int prefill_args(const void* q, int64_t q_stride_token, int64_t q_stride_head,
                         const void* k_cache, const void* v_cache, int64_t kv_stride_slot,
                         int64_t kv_stride_head, const int32_t* indices, const int32_t* qo_indptr,

@@ -700,6 +700,26 @@ def test_prefill_every_tile_once(oracle, dev, hq, hkv):
     check_prefill(oracle, dev, b, hq, hkv, 23, f"prefill tiles {hq}/{hkv}")
 
 
+@pytest.mark.parametrize("hq,hkv,new", [
+    # mean length exactly 0.9 of the longest (the tiles go rank by rank), just below
+    # it, equal lengths in 128-row tiles and odd counts of them, many requests
+    (16, 8, [100, 80]), (16, 8, [100, 79]), (16, 2, [320] * 5), (8, 1, [129, 130, 128]),
+    (12, 6, [201] * 11), (32, 8, [1, 1, 1]), (16, 16, [77] * 9), (64, 4, [66, 60, 57, 64]),
+    (8, 8, [4, 0, 5, 5, 5, 5, 5, 5, 5, 5, 5]),
+    (32, 8, [33] * 95), (32, 8, [33] * 97),  # 1520 items, 1552 (past the limit)
+])
+def test_prefill_even_lengths(oracle, dev, hq, hkv, new):
+    """Batches of like lengths: each tile is some workgroup's either way the
+    items are numbered (the output starts as NaN)."""
+    note(f"prefill even lengths hq={hq} hkv={hkv} {new}")
+    cached = [3 * (i % 3) for i in range(len(new))]
+    b = wl.make_paged_batch(np.random.default_rng(hkv), cached,
+                            [n + c for n, c in zip(new, cached)], page_size=16)
+    if 0 in new:  # a request with neither query tokens nor work
+        b.qo_indptr[:] = np.concatenate([[0], np.cumsum(new)])
+    check_prefill(oracle, dev, b, hq, hkv, 24, f"prefill even {hq}/{hkv}")
+
+
 @pytest.mark.parametrize("hq,hkv,cached,new", [
     (32, 8, [2000, 9001, 500, 0], [17, 90, 33, 40]),  # shares beside whole tiles
     (16, 8, [4095], [2]),                             # one wave of rows
