@@ -694,7 +694,7 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     u32x4_t kt[kSmallWaves][256];
     float xch[34][kSmallWaves][kWave];
   } xs;
-  __shared__ int32_t locs[kMaxLayerBatch];
+  __shared__ __attribute__((aligned(16))) int32_t locs[kMaxLayerBatch];
   __shared__ uint64_t shared_rows;  // requests whose new slot is among this one's slots (see new_token)
   auto& xch = xs.xch;
   const int h = blockIdx.x;
@@ -716,7 +716,8 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
     }
     new_pos = nt.positions[r];
     new_loc = nt.out_loc[r];
-    if (static_cast<int>(threadIdx.x) < a.batch) locs[threadIdx.x] = nt.out_loc[threadIdx.x];
+    if (threadIdx.x < kMaxLayerBatch)  // past the batch: matches no other slot
+      locs[threadIdx.x] = static_cast<int>(threadIdx.x) < a.batch ? nt.out_loc[threadIdx.x] : new_loc;
     if (threadIdx.x == 0) shared_rows = 0;
   }
   const int total = a.kv_indptr[a.batch];
@@ -770,10 +771,21 @@ __global__ void __launch_bounds__(kSmallWaves * kWave) paged_decode_small_kernel
         const int slot = sp[e];
         if (slot == new_loc) {
           if (e != len - 1) seen |= 1ull << r;  // its own slot, not in its usual place
-        } else {
-          for (int o = 0; o < a.batch; ++o)
-            if (locs[o] == slot) seen |= 1ull << o;
+          continue;
         }
+        // Eight of the batch's new slots a turn, and which of them only on a hit:
+        // one at a time was 2.7 us of 23.2 for 64 requests, one of them of 1400
+        // tokens (16q/1kv).
+        bool hit = false;
+        for (int o = 0; a.batch > 1 && o < a.batch; o += 8) {
+          const u32x4_t l0 = *reinterpret_cast<const u32x4_t*>(locs + o);
+          const u32x4_t l1 = *reinterpret_cast<const u32x4_t*>(locs + o + 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) hit |= (l0[i] == static_cast<uint32_t>(slot)) | (l1[i] == static_cast<uint32_t>(slot));
+        }
+        if (!hit) continue;
+        for (int o = 0; o < a.batch; ++o)
+          if (locs[o] == slot) seen |= 1ull << o;
       }
       if (seen != 0) atomicOr(reinterpret_cast<unsigned long long*>(&shared_rows), seen);
     }

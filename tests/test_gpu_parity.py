@@ -1098,6 +1098,26 @@ def test_decode_layer_equals_store_then_decode(dev, hq, hkv, lens, norm, unknown
         assert torch.equal(got.contiguous().view(torch.int16), ref.contiguous().view(torch.int16)), what
 
 
+def _graph_us(fn, n=50):
+    """us of fn, best of ten replays of a graph of n."""
+    fn()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        for _ in range(n):
+            fn()
+    best = float("inf")
+    for _ in range(10):
+        t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        t0.record()
+        graph.replay()
+        t1.record()
+        torch.cuda.synchronize()
+        best = min(best, t0.elapsed_time(t1) * 1000 / n)
+    return best
+
+
 def test_decode_layer_padding_rows_cost_like_others(dev):
     """Rows that share one spare slot (a padded batch's dummies) do not store
     for each other: 32 of them take about as long as 32 rows with slots of
@@ -1113,27 +1133,33 @@ def test_decode_layer_padding_rows_cost_like_others(dev):
     def once(l, i):
         capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, l, 1e-6, i, kvp, hq, o, ws)
 
-    def us(l, i):
-        once(l, i)
-        side = torch.cuda.Stream()
-        side.wait_stream(torch.cuda.current_stream())
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=side):
-            for _ in range(50):
-                once(l, i)
-        best = float("inf")
-        for _ in range(10):
-            t0, t1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
-            t0.record()
-            graph.replay()
-            t1.record()
-            torch.cuda.synchronize()
-            best = min(best, t0.elapsed_time(t1) * 1000 / 50)
-        return best
-
-    own, shared = us(loc, idx), us(shared_loc, shared_idx)
+    own = _graph_us(lambda: once(loc, idx))
+    shared = _graph_us(lambda: once(shared_loc, shared_idx))
     print(f"[case] own slots {own:.2f} us, one slot {shared:.2f} us", flush=True)
     assert shared < 1.5 * own + 1.0
+
+
+def test_decode_layer_of_many_requests_is_no_slower_than_its_parts(dev):
+    """The look for the batch's new slots among a long request's: 64 requests, one
+    of 1400 tokens, in the layer's launch and as store pass and decode."""
+    note("decode layer, 64 requests, time against its parts")
+    hq, hkv, lens = 16, 1, [1400] + [300] * 63
+    plan, qkv, kc, vc, (qw, kw), cos, sin, pos, loc, idx, kvp = _decode_layer_case(
+        dev, hq, hkv, lens, True, 46, unknown=True)
+    ws = capi.decode_workspace(plan, dev)
+    o = torch.zeros((len(lens), hq, 128), device=dev, dtype=torch.bfloat16)
+    q = qkv[:, :hq * 128].view(len(lens), hq, 128)
+
+    def parts():
+        capi.fused_qknorm_rope_store(qkv, kc, vc, qw, kw, cos, sin, pos, loc, hq, hkv, 128, 1e-6,
+                                     write_k_back=False)
+        capi.paged_decode(plan, q, kc, vc, idx, kvp, o, ws, 1 / math.sqrt(128))
+
+    two = _graph_us(parts)
+    one = _graph_us(lambda: capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, loc, 1e-6,
+                                              idx, kvp, hq, o, ws))
+    print(f"[case] store and decode {two:.2f} us, layer {one:.2f} us", flush=True)
+    assert one < 1.08 * two
 
 
 @pytest.mark.parametrize("lens", [[300, 200], [900, 3]])  # one launch, two
