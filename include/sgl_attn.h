@@ -283,7 +283,8 @@ int sgl_decode_plan_check(const sgl_decode_plan_t* plan, const int32_t* kv_indpt
  * head, request), or per (kv head, unit) when the batch has more requests
  * than the plan has units), or one for small batches
  * (plans at the 64-token minimum unit with batch_size x Hkv workgroups at
- * most the CU count and no request longer than 800 tokens). Calls that share one workspace must be stream-ordered.
+ * most the CU count and no request longer than 800 tokens, 896, 1024 and 1152 from
+ * 8, 16 and 64 of these workgroups). Calls that share one workspace must be stream-ordered.
  * Replaces: BatchDecodeWithPagedKVCacheDispatched call in
  *           FlashInferBackend::forward (src/attention/flashinfer_backend.cu:553-595).
  */

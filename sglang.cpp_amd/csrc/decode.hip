@@ -641,12 +641,18 @@ __global__ void __launch_bounds__(512, 1) mixed_attention_kernel(DecodeArgs d, p
 // two steps in flight measured 389 -> 408 us (28 layers, four requests of 380 to
 // 640 tokens), two steps to a chain as well 434 us.
 constexpr int kSmallWaves = 8;
-// A request's workgroup streams about 46 GB/s of K/V, the launch pair costs
-// the same for any length: per layer (store included, 32q/8kv, one request, a
-// captured step) 11.2, 14.0, 16.9, 19.8 and 54 us here at 256, 512, 768, 1024
-// and 4096 tokens against 17.1, 17.4, 17.5, 17.6 and 18.6 us; four requests 12.3,
-// 15.1, 18.1, 21.0 and 56 against 18.1, 18.4, 18.6, 19.2 and 24.7.
-constexpr int kSmallLongest = 800;
+// The longest request the kernel takes. Its time grows with that request, about
+// 46 GB/s of K/V a workgroup; the launch pair's hardly does, but with the
+// workgroups of its two launches. Per layer, store included (32q/8kv, pools past
+// the last-level cache), here and there, us, at 500, 700, 816, 1000, 1400 tokens:
+// one request 11.8, 13.9, 15.3, 17.4, 21.8 and 15.8, 16.3, 16.8, 16.6, 16.5; four
+// 12.2, 14.7, 16.2, 18.4, 23.4 and 19.1, 19.2, 19.8, 20.4, 19.7; sixteen (to 1000)
+// 14.0, 17.9, 19.9, 22.2 and 21.3, 23.1, 23.6, 26.0.
+// One request of 850 tokens of 4 and 2 heads 14.6 and 14.0 against 13.9 and 12.6; 64
+// requests, one of them of 1100 (16q/2kv), 18.0 against 19.6.
+constexpr int small_longest(int64_t workgroups) {
+  return workgroups < 8 ? 800 : workgroups < 16 ? 896 : workgroups < 64 ? 1024 : 1152;
+}
 constexpr int kSmallStage = 8192;  // slot indices staged in LDS (longer requests read them from HBM)
 
 // The new token of each request, for the variant that normalises, rotates and
@@ -1386,8 +1392,10 @@ void bind_workspace(DecodeArgs& a, const sgl_decode_plan_t* plan, void* workspac
 
 // Decode launch + merge launch on one stream (or the small-batch kernel alone).
 bool small_batch(const DecodeArgs& a, const sgl_decode_plan_t* plan) {
-  return plan->kv_chunk_size <= kMinUnit && plan->max_request_tokens <= kSmallLongest &&
-         static_cast<int64_t>(a.batch) * a.hkv <= static_cast<int64_t>(device_cu_count());
+  const int64_t wgs = static_cast<int64_t>(a.batch) * a.hkv;
+  return plan->kv_chunk_size <= kMinUnit &&
+         plan->max_request_tokens <= small_longest(wgs) &&
+         wgs <= static_cast<int64_t>(device_cu_count());
 }
 
 int launch_decode(const DecodeArgs& a, const sgl_decode_plan_t* plan, hipStream_t s) {

@@ -219,7 +219,7 @@ def test_attention_layer_matches_unfused_modules(dev, sb):
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("hq,hkv,lens", [
     (16, 8, [512, 400, 1, 17]),        # one launch
-    (32, 8, [801, 30]),                # two: a long request
+    (32, 8, [1025, 30]),               # two: a long request
     (32, 4, [60 + i for i in range(65)]),  # two: past the one-launch batch
 ])
 def test_attention_layer_decode_matches_store_then_attend(dev, sb, hq, hkv, lens, norm):

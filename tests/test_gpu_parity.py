@@ -468,7 +468,9 @@ def test_decode_small_batch_kernel(oracle, dev, hq, hkv, lens):
     note(f"decode small-batch kernel hq={hq} hkv={hkv} lens={lens}")
     rng = np.random.default_rng(27)
     b = wl.make_paged_batch(rng, [max(x - 1, 0) for x in lens], lens, page_size=16, decode=True)
-    q, kc, vc, o, scale, plan = run_decode(dev, b, hq, hkv, 128, 28)
+    plan = capi.decode_plan(b.kv_indptr, hq, hkv, 128)
+    plan.max_request_tokens = 0  # whatever the lengths
+    q, kc, vc, o, scale, _ = run_decode(dev, b, hq, hkv, 128, 28, plan=plan)
     assert plan.kv_chunk_size == 64 and plan.batch_size * hkv <= 256
     ref = oracle.decode(u16(q).copy(), u16(kc), u16(vc), b.indices, b.kv_indptr, scale)
     assert_attn_close(o.float().cpu().numpy(), ref, what="small-batch decode")
@@ -476,7 +478,11 @@ def test_decode_small_batch_kernel(oracle, dev, hq, hkv, lens):
 
 @pytest.mark.parametrize("unknown_longest", [False, True])
 @pytest.mark.parametrize("hq,hkv,lens", [
-    (32, 8, [800]), (32, 8, [801]),  # either side of the one-launch limit
+    (32, 8, [800]), (32, 8, [801]),
+    (32, 4, [800]), (32, 4, [801]),  # either side of the one-launch limit: 4 workgroups,
+    (32, 8, [896]), (32, 8, [897]),  # 8,
+    (16, 8, [1024, 9]), (16, 8, [1025, 9]), (16, 1, [1024] * 15), (16, 1, [1025] * 16),  # 15, 16
+    (8, 8, [1152] + [9] * 7), (8, 8, [1153] + [9] * 7), (8, 1, [1152] + [8] * 62),  # 64, 63
     (16, 8, [1024]), (16, 8, [1023, 9]),  # 16 units: the fold for few long requests, and not
     (32, 8, [12001]), (64, 4, [5000, 3000]), (8, 8, [4097]), (8, 1, [9000]),
 ])
@@ -1055,7 +1061,10 @@ def _decode_layer_case(dev, hq, hkv, lens, norm, seed, unknown=False, alias=None
     (16, 8, [512, 400, 1, 17], True, False, None, None),
     (16, 8, [512, 400, 1, 17], False, False, None, None),
     (32, 8, [800], True, False, None, None),
-    (32, 8, [801, 3], True, False, None, None),            # two launches
+    (32, 8, [801, 3], True, False, None, None),
+    (32, 8, [896], True, False, None, None),
+    (32, 8, [1024, 3], True, False, None, None),
+    (32, 8, [1025, 3], True, False, None, None),           # two launches
     (64, 4, [16, 15, 33], True, False, None, None),        # G = 16
     (8, 8, [64, 0, 65], True, False, None, None),          # an empty request
     (8, 1, [9000, 5], True, True, None, None),             # slots past the LDS stage
@@ -1162,7 +1171,7 @@ def test_decode_layer_of_many_requests_is_no_slower_than_its_parts(dev):
     assert one < 1.08 * two
 
 
-@pytest.mark.parametrize("lens", [[300, 200], [900, 3]])  # one launch, two
+@pytest.mark.parametrize("lens", [[300, 200], [1100, 3]])  # one launch, two
 def test_decode_layer_error_leaves_its_inputs(dev, lens):
     """A refused call writes nothing."""
     note(f"decode layer refused {lens}")
