@@ -979,8 +979,17 @@ __global__ void __launch_bounds__(kMaxGroup * (kD / 4)) decode_merge_kernel(Deco
 // flight at a time, and lane group 0 folds the groups through LDS. What bounds
 // it is the chain of dependent load rounds: 188 pieces are 3 rounds here and
 // 47 in the kernel above.
+// A plan's units are its capacity: a captured step of short requests has few
+// pieces each, and lane group 0 folds up to kFewPieces by itself (decode of four
+// requests of 100 tokens, 32q/8kv, units for 40,960 each, us: the kernel above
+// 14.4, all groups here 15.5, one 14.5; at 2000 tokens 19.9 above, 17.2 here).
 constexpr int kLongGroups = 16;
-constexpr int kLongPieces = 16;  // mean pieces per request from which this kernel is used
+constexpr int kFewPieces = 8;
+// Units per request from which this kernel is used, and the (head, request)
+// workgroups below which it is: 1024 of them fill the device once, and then their
+// launch shows (64q/4kv, 16 requests of 500 tokens 18.3 against 16.8 above).
+constexpr int kLongPieces = 16;
+constexpr int64_t kLongWorkgroups = 1024;
 
 __global__ void __launch_bounds__(kLongGroups * 32) decode_merge_long_kernel(DecodeArgs a) {
   __shared__ float xch[kLongGroups][6][32];
@@ -1003,7 +1012,9 @@ __global__ void __launch_bounds__(kLongGroups * 32) decode_merge_long_kernel(Dec
   if (u0 == u1) return;  // whole request, written by the decode kernel
   const int s0 = 2 * u0 + (rb > u0 * W ? 1 : 0);
   const int np = u1 - u0 + 1;
-  const int per = (np + kLongGroups - 1) / kLongGroups;
+  const bool few = np <= kFewPieces;
+  if (few && grp != 0) return;
+  const int per = few ? np : (np + kLongGroups - 1) / kLongGroups;
   const int c1 = min(np, (grp + 1) * per);
   float m = -INFINITY, den = 0.f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -1034,6 +1045,12 @@ __global__ void __launch_bounds__(kLongGroups * 32) decode_merge_long_kernel(Dec
       den += wgt;
       acc += v[k] * wgt;
     }
+  }
+  if (few) {
+    const float inv = den > 0.f ? 1.0f / den : 0.f;
+    *reinterpret_cast<u32x2_t*>(op) =
+        u32x2_t{pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
+    return;
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) xch[grp][i][lane] = acc[i];
@@ -1367,7 +1384,8 @@ void launch_merge(const DecodeArgs& a, hipStream_t s) {
   if (a.batch > a.num_units + 1)
     hipLaunchKernelGGL(decode_merge_units_kernel, dim3(a.hkv, a.num_units + 1),
                        dim3(merge_threads(a.group)), 0, s, a);
-  else if (a.num_units >= kLongPieces * static_cast<int64_t>(a.batch))
+  else if (a.num_units >= kLongPieces * static_cast<int64_t>(a.batch) &&
+           static_cast<int64_t>(a.batch) * a.hq < kLongWorkgroups)
     hipLaunchKernelGGL(decode_merge_long_kernel, dim3(a.hq, a.batch), dim3(kLongGroups * 32), 0, s,
                        a);
   else

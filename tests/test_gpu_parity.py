@@ -530,6 +530,24 @@ def test_decode_long_fold_keeps_infinities(dev, hq, hkv, n):
                       what="the finite columns")
 
 
+@pytest.mark.parametrize("hq,hkv,lens", [
+    # pieces of 64 tokens: one, two, either side of the 8 one lane group folds, more
+    (32, 8, [64, 65, 512, 513, 576, 577, 1]), (16, 8, [1, 3000]), (32, 4, [500] * 16),
+    (64, 4, [700, 40, 0, 130] + [300] * 11), (64, 4, [700, 40, 0, 130] + [300] * 12),  # 960, 1024
+])
+def test_decode_short_requests_of_a_large_plan(oracle, dev, hq, hkv, lens):
+    """A plan made for 40,960 tokens a request (a captured step) with requests
+    of a few pieces each: the fold for many units."""
+    note(f"decode short requests, large plan hq={hq} hkv={hkv} lens={lens}")
+    plan = capi.decode_plan(np.arange(len(lens) + 1, dtype=np.int32) * 40960, hq, hkv, 128)
+    assert plan.num_units >= 16 * len(lens) and plan.kv_chunk_size > 64
+    b = wl.make_paged_batch(np.random.default_rng(34), [max(0, x - 1) for x in lens], lens,
+                            page_size=16, decode=True)
+    q, kc, vc, o, scale, _ = run_decode(dev, b, hq, hkv, 128, 33, plan=plan)
+    ref = oracle.decode(u16(q).copy(), u16(kc), u16(vc), b.indices, b.kv_indptr, scale)
+    assert_attn_close(o.float().cpu().numpy(), ref, what="short requests of a large plan")
+
+
 def test_decode_few_long_requests_past_the_plan(dev):
     """A long request past the plan's capacity: NaN rows and the status."""
     note("decode long request past its plan")
