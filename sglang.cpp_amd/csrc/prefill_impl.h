@@ -34,7 +34,7 @@ struct PrefillArgs {
   int64_t o_st, o_sh;
   int tiles_per_req;  // query tiles (or pairs) per (request, kv head)
   int num_kv_heads;
-  int batch, even_tokens;  // unpaired launches, see unpaired_items
+  int batch, even_tokens, ranks, xcd_shift;  // unpaired launches, see unpaired_items
   // Planned launches (prefill_item kList): item lin / Hkv = {request, first
   // packed row << 4 | waves of rows, first kv tile, end kv tile | kPartial}, kv
   // head lin % Hkv; partial items leave their state in part[lin].
@@ -374,14 +374,19 @@ constexpr int prefill_lds_bytes() {
 // often (at 0.75, 32q/8kv, 2 requests up to 4096 tokens: 196 us against 241),
 // and so it is for many items, whose last ones weigh little (64q/4kv, 12 x 700
 // tokens, 2112 items: 167 against 191; 16q/16kv, 16 x 1000 behind 2048, 2048
-// items: 419 against 471).
+// items: 419 against 471). Three and more requests in 128-row tiles that are all
+// resident at once (512 items, two a CU) gain from 0.75 on (16q/8kv, four of up to
+// 1000 tokens, 37.4 against 30.2; 8q/8kv, four of up to 1500, 46 against 38).
 inline int64_t unpaired_items(PrefillArgs& a, int max_qo, int tile_rows, int batch) {
   const int H = a.num_kv_heads;
   const int64_t m = H < kXcds && kXcds % H == 0 ? kXcds / H : 1;
   const int64_t tiles = (static_cast<int64_t>(max_qo) * a.group + tile_rows - 1) / tile_rows;
   const int64_t per_req = (tiles + m - 1) / m * m, items = per_req * H * batch;
-  const int64_t even = (9 * static_cast<int64_t>(max_qo) * batch + 9) / 10;
+  const int64_t percent = tile_rows == 128 && batch > 2 && items <= 512 ? 75 : 90;
+  const int64_t even = (percent * max_qo * batch + 99) / 100;
   a.tiles_per_req = static_cast<int>(per_req);
+  a.ranks = static_cast<int>(per_req / m);
+  a.xcd_shift = __builtin_ctz(static_cast<unsigned>(m));  // m: a power of two
   a.batch = batch;
   a.even_tokens = batch > 1 && items <= 1536 && even < 0x7fffffff ? static_cast<int>(even) : 0x7fffffff;
   return items;
@@ -390,30 +395,27 @@ inline int64_t unpaired_items(PrefillArgs& a, int max_qo, int tile_rows, int bat
 // Request, kv head and query tile of item `lin` of an unpaired launch
 // (batch x Hkv x tiles_per_req items).
 __device__ __forceinline__ void item_of(const PrefillArgs& a, int lin, int& r, int& h, int& tile) {
-  const int H = a.num_kv_heads;
-  int j, m = 1, x = 0;
-  if (H < kXcds && kXcds % H == 0) {
-    m = kXcds / H;  // XCDs per head, consecutive ones
-    x = lin % kXcds;
+  int j, x = 0;
+  if (a.xcd_shift != 0) {  // a head's tiles on 2, 4 or 8 consecutive XCDs
     j = lin / kXcds;
-    h = x / m;
-    x -= h * m;
+    h = (lin % kXcds) >> a.xcd_shift;
+    x = (lin % kXcds) - (h << a.xcd_shift);
   } else {
     // Multiples of 8 heads: head h on XCD h % 8. Other counts: the same
     // order, the heads wherever they fall.
-    j = lin / H;
-    h = lin - j * H;
+    j = lin / a.num_kv_heads;
+    h = lin - j * a.num_kv_heads;
   }
-  const int ranks = a.tiles_per_req / m;
   int rank;
-  if (a.qo_indptr[a.batch] - a.qo_indptr[0] >= a.even_tokens) {
+  if (a.even_tokens != 0x7fffffff &&  // else no load in front of the request's own
+      a.qo_indptr[a.batch] - a.qo_indptr[0] >= a.even_tokens) {
     rank = j / a.batch;
     r = j - rank * a.batch;
   } else {
-    r = j / ranks;
-    rank = j - r * ranks;
+    r = j / a.ranks;
+    rank = j - r * a.ranks;
   }
-  tile = a.tiles_per_req - 1 - (rank * m + x);
+  tile = a.tiles_per_req - 1 - ((rank << a.xcd_shift) + x);
 }
 
 // kList = true (W = 8, KS = 1): the items and their kv shares come from a

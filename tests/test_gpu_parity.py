@@ -725,12 +725,13 @@ def test_prefill_every_tile_once(oracle, dev, hq, hkv):
 
 
 @pytest.mark.parametrize("hq,hkv,new", [
-    # mean length exactly 0.9 of the longest (the tiles go rank by rank), just below
+    # mean length exactly 0.9 of the longest (the tiles go rank by rank), below
     # it, equal lengths in 128-row tiles and odd counts of them, many requests
     (16, 8, [100, 80]), (16, 8, [100, 79]), (16, 2, [320] * 5), (8, 1, [129, 130, 128]),
     (12, 6, [201] * 11), (32, 8, [1, 1, 1]), (16, 16, [77] * 9), (64, 4, [66, 60, 57, 64]),
     (8, 8, [4, 0, 5, 5, 5, 5, 5, 5, 5, 5, 5]),
     (32, 8, [33] * 95), (32, 8, [33] * 97),  # 1520 items, 1552 (past the limit)
+    (16, 8, [300, 200, 175]), (16, 8, [300, 200, 174]),  # 0.75 of the longest, below it
 ])
 def test_prefill_even_lengths(oracle, dev, hq, hkv, new):
     """Batches of like lengths: each tile is some workgroup's either way the
