@@ -379,14 +379,14 @@ constexpr int prefill_lds_bytes() {
 // 1000 tokens, 37.4 against 30.2; 8q/8kv, four of up to 1500, 46 against 38).
 inline int64_t unpaired_items(PrefillArgs& a, int max_qo, int tile_rows, int batch) {
   const int H = a.num_kv_heads;
-  const int64_t m = H < kXcds && kXcds % H == 0 ? kXcds / H : 1;
+  const int64_t m = H <= kXcds && kXcds % H == 0 ? kXcds / H : 1;
   const int64_t tiles = (static_cast<int64_t>(max_qo) * a.group + tile_rows - 1) / tile_rows;
   const int64_t per_req = (tiles + m - 1) / m * m, items = per_req * H * batch;
   const int64_t percent = tile_rows == 128 && batch > 2 && items <= 512 ? 75 : 90;
   const int64_t even = (percent * max_qo * batch + 99) / 100;
   a.tiles_per_req = static_cast<int>(per_req);
   a.ranks = static_cast<int>(per_req / m);
-  a.xcd_shift = __builtin_ctz(static_cast<unsigned>(m));  // m: a power of two
+  a.xcd_shift = H <= kXcds && kXcds % H == 0 ? __builtin_ctz(static_cast<unsigned>(m)) : -1;
   a.batch = batch;
   a.even_tokens = batch > 1 && items <= 1536 && even < 0x7fffffff ? static_cast<int>(even) : 0x7fffffff;
   return items;
@@ -395,27 +395,36 @@ inline int64_t unpaired_items(PrefillArgs& a, int max_qo, int tile_rows, int bat
 // Request, kv head and query tile of item `lin` of an unpaired launch
 // (batch x Hkv x tiles_per_req items).
 __device__ __forceinline__ void item_of(const PrefillArgs& a, int lin, int& r, int& h, int& tile) {
-  int j, x = 0;
-  if (a.xcd_shift != 0) {  // a head's tiles on 2, 4 or 8 consecutive XCDs
-    j = lin / kXcds;
-    h = (lin % kXcds) >> a.xcd_shift;
-    x = (lin % kXcds) - (h << a.xcd_shift);
+  // The smallest launches wait for this: no division for head counts that
+  // divide the XCDs, none for a single request, no load that does not decide.
+  uint32_t j, x = 0;
+  const uint32_t l = static_cast<uint32_t>(lin);
+  int shift = a.xcd_shift;
+  if (shift >= 0) {  // a head's tiles on 2^shift consecutive XCDs
+    j = l / kXcds;
+    const uint32_t xcd = l % kXcds;
+    h = static_cast<int>(xcd >> shift);
+    x = xcd - (static_cast<uint32_t>(h) << shift);
   } else {
     // Multiples of 8 heads: head h on XCD h % 8. Other counts: the same
     // order, the heads wherever they fall.
-    j = lin / a.num_kv_heads;
-    h = lin - j * a.num_kv_heads;
+    j = l / static_cast<uint32_t>(a.num_kv_heads);
+    h = static_cast<int>(l - j * a.num_kv_heads);
+    shift = 0;
   }
-  int rank;
-  if (a.even_tokens != 0x7fffffff &&  // else no load in front of the request's own
-      a.qo_indptr[a.batch] - a.qo_indptr[0] >= a.even_tokens) {
-    rank = j / a.batch;
-    r = j - rank * a.batch;
-  } else {
-    r = j / a.ranks;
-    rank = j - r * a.ranks;
+  uint32_t rank = j;
+  r = 0;
+  if (a.batch > 1) {
+    if (a.even_tokens != 0x7fffffff &&
+        a.qo_indptr[a.batch] - a.qo_indptr[0] >= a.even_tokens) {
+      rank = j / static_cast<uint32_t>(a.batch);
+      r = static_cast<int>(j - rank * a.batch);
+    } else {
+      r = static_cast<int>(j / static_cast<uint32_t>(a.ranks));
+      rank = j - static_cast<uint32_t>(r) * a.ranks;
+    }
   }
-  tile = a.tiles_per_req - 1 - ((rank << a.xcd_shift) + x);
+  tile = a.tiles_per_req - 1 - static_cast<int>((rank << shift) + x);
 }
 
 // kList = true (W = 8, KS = 1): the items and their kv shares come from a
@@ -529,11 +538,12 @@ __device__ __forceinline__ void prefill_item(PrefillArgs a, char* lds_raw, int l
     return (min(kv_len, last_row / G + off + 1) + kBN - 1) / kBN;
   };
   const int ntiles = tiles_for(kList ? row0 : tile0 * kGM);
-  // A wave past the request's last row only gathers. Not in the unpaired 8-wave
-  // launches: few of their tiles are short, and the test in each step cost the
-  // mixed launch 1 to 2% (64 decode rows of 1024 to 32768 tokens beside a chunk of
-  // 2048, 32q/4kv, 320 -> 314 us).
-  constexpr bool kSkipWaves = kPair || kList || W < 8;
+  // A wave past the request's last row only gathers, where that pays for a test in
+  // each step: not in the unpaired 8-wave launches, few of whose tiles are short
+  // (64 decode rows of 1024 to 32768 tokens beside a chunk of 2048, 32q/4kv, 320 ->
+  // 314 us without it), and not in the split-kv ones (500 new tokens on 500 cached,
+  // 32q/8kv, 21.2 -> 20.3).
+  constexpr bool kSkipWaves = kPair || kList || (W < 8 && KS == 1);
   const int my_tiles = !kPair ? (row0 + gwave * 32 < row_end ? ntiles : 0)
                        : !grp_rows ? 0 : row0 == tile0 * kGM ? ntiles : tiles_for(row0);
   // First token index at which some row of the group may be masked.
