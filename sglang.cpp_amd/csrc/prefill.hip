@@ -40,7 +40,9 @@ namespace {
 // were set where both routes were timed: 500 new tokens on 3000 cached 63 -> 50
 // us a layer, 100 on 1500 34 -> 23, 512 on 1000 (16q/8kv) 35 -> 30, while
 // 1000 tokens without a prefix (34 us, planned 40) and 100 on 500 (20 and 20)
-// stay unplanned.
+// stay unplanned. Over 111 batches that are planned (2 to 600 new tokens on 64 to
+// 16,000, up to 16 requests, twelve head layouts) the planned route takes 0.45 of
+// the other's time on average and was the slower one once, by 4%.
 constexpr int32_t kStepCost[9] = {0, 14, 14, 15, 15, 20, 22, 24, 27};
 constexpr int64_t kStateCost = 2;
 constexpr int64_t kMinShare = 60;
