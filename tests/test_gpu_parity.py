@@ -1187,7 +1187,7 @@ def test_decode_layer_of_many_requests_is_no_slower_than_its_parts(dev):
     one = _graph_us(lambda: capi.decode_layer(plan, qkv, kc, vc, qw, kw, cos, sin, pos, loc, 1e-6,
                                               idx, kvp, hq, o, ws))
     print(f"[case] store and decode {two:.2f} us, layer {one:.2f} us", flush=True)
-    assert one < 1.08 * two
+    assert one < 1.1 * two  # 1.02; 1.16 with one slot compared at a time
 
 
 @pytest.mark.parametrize("lens", [[300, 200], [1100, 3]])  # one launch, two
